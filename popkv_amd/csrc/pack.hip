@@ -1,22 +1,16 @@
 // Key prepack and per-token append of PopKV retrieval metadata (gfx950).
 //
-// head_dim 128 (pack128_kernel, the encode itself pack128_group in
-// pack128.h): one workgroup per (KV head, token group), one wave per chunk
-// of max(G, 32) dimensions (2 or 4 waves).
-//   Phase 1 -- lane l owns dims 2l and 2l+1; the waves stream interleaved
-//              rows of the group with coalesced 4-byte loads (256 bytes per
-//              wave instruction), keeping per-dimension min/max in registers;
-//              the partial extrema meet in LDS and the thresholds
-//              0.5*max / 0.5*min go to LDS.
-//   Phase 2 -- one token per lane, each wave on its dimension chunk: the
-//              lane re-reads its slice of the row (a cache hit), forms the
-//              sign/magnitude words and reduces its representatives in
-//              registers in the production tree order (G64 pairs dims j and
-//              j+32 first), then writes its words and fp16 representatives.
-// No cross-lane shuffles are needed for the bit-exact sums: the tree lives in
-// one lane's registers.  Other head sizes (pack_kernel) use 256 threads per
-// group: per-dimension extrema by (dimension, token stripe), then one token
-// per thread.
+// head_dim 128, token groups of 8 .. 128 (powers of two): pack128_block_kernel
+// (pack128_block in pack128.h), one workgroup per 64 rows (128 for 128-token
+// groups).  Other group sizes and the append: pack128_kernel, one workgroup
+// per (KV head, token group), one wave per chunk of max(G, 32) dimensions
+// (pack128_group in pack128.h).  In both, the extrema of each dimension over
+// its token group come first (thresholds 0.5*max / 0.5*min in LDS), then one
+// token per lane: the sign/magnitude words and the representatives, reduced
+// in one lane's registers in the production tree order, so the bit-exact
+// sums need no cross-lane shuffles.  Other head sizes (pack_kernel) use 256
+// threads per group: per-dimension extrema by (dimension, token stripe),
+// then one token per thread.
 //
 // Semantics follow the reference packers: popkv_ext.cu:79-143 (G32),
 // :376-500 (fused G16/G64, head_dim 128), :283-374 (generic G16/G64), with
@@ -190,7 +184,8 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
 
 // Prefix prepack (APPEND false): block (x, y) encodes token group x of KV
 // head y, rows [x*tg, min(x*tg + tg, tokens)) of `keys`, into packed rows
-// y*cap + offset + x*tg + t.  Fused append (APPEND true): block i appends
+// y*cap + offset + x*tg + t, for the group sizes pack128_block does not
+// take.  Fused append (APPEND true): block i appends
 // the new token of (sequence, KV head) i (pack128_append).  STAGE (16-bit
 // rows; tg <= 64 at G 64, tg <= 128 at G 32 / G 16): the group's rows are
 // read from memory once, into LDS, and the encode pass reads them there.
@@ -220,6 +215,33 @@ __global__ __launch_bounds__(kWave * pack128_waves<G>()) void pack128_kernel(
     }
 }
 
+// Prefix prepack for token groups of TG = 8 .. 128: block (x, y) encodes rows
+// [ROWS x, ROWS x + ROWS) of KV head y (pack128_block).
+template <typename T, int G, int TG, bool STAGE>
+__global__ __launch_bounds__((pack128_block_threads<G, TG>())) void pack128_block_kernel(
+    const T* __restrict__ keys, int64_t head_stride, int64_t tokens, int32_t* __restrict__ k_sign,
+    int32_t* __restrict__ k_mag, uint16_t* __restrict__ k_low, uint16_t* __restrict__ k_delta, int64_t cap,
+    int64_t offset) {
+    args_in_sgprs(keys, head_stride, tokens, k_sign, k_mag, k_low, k_delta, cap, offset);
+    const int64_t kvh = blockIdx.y;
+    const int64_t gs = static_cast<int64_t>(blockIdx.x) * pack128_block_rows(TG);
+    const int n = static_cast<int>(min(static_cast<int64_t>(pack128_block_rows(TG)), tokens - gs));
+    pack128_block<T, G, TG, STAGE>(keys + kvh * head_stride + gs * 128, n, kvh * cap + offset + gs, k_sign, k_mag,
+                                   k_low, k_delta);
+}
+
+template <typename T, int G, int TG>
+hipError_t launch_pack_block(const T* keys, int64_t kvh, int64_t tokens, int64_t head_stride, int32_t* ks, int32_t* km,
+                             uint16_t* kl, uint16_t* kd, int64_t cap, int64_t off, hipStream_t stream) {
+    constexpr int rows = pack128_block_rows(TG);
+    const dim3 grid(static_cast<unsigned>((tokens + rows - 1) / rows), static_cast<unsigned>(kvh));
+    const dim3 block(pack128_block_threads<G, TG>());
+    constexpr bool kStage = sizeof(T) == 2 || TG <= 64;
+    hipLaunchKernelGGL((pack128_block_kernel<T, G, TG, kStage>), grid, block, 0, stream,
+                       keys, head_stride, tokens, ks, km, kl, kd, cap, off);
+    return hipGetLastError();
+}
+
 template <typename T, int G>
 hipError_t launch_pack_t(const T* keys, int64_t kvh, int64_t tokens, int d, int64_t head_stride,
                          int32_t* ks, int32_t* km, uint16_t* kl, uint16_t* kd, int64_t cap, int64_t off,
@@ -231,6 +253,18 @@ hipError_t launch_pack_t(const T* keys, int64_t kvh, int64_t tokens, int d, int6
                       (reinterpret_cast<uintptr_t>(ks) % 16 == 0) && (reinterpret_cast<uintptr_t>(km) % 16 == 0) &&
                       (reinterpret_cast<uintptr_t>(kl) % 16 == 0) && (reinterpret_cast<uintptr_t>(kd) % 16 == 0);
     constexpr bool kStageable = sizeof(T) == 2;
+    // the block form wherever the groups fill its rows: it is faster at every
+    // preset (figures at pack128_block)
+    if (fast) {
+        switch (tg) {
+            case 8: return launch_pack_block<T, G, 8>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);
+            case 16: return launch_pack_block<T, G, 16>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);
+            case 32: return launch_pack_block<T, G, 32>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);
+            case 64: return launch_pack_block<T, G, 64>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);
+            case 128: return launch_pack_block<T, G, 128>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);
+            default: break;  // any other size: one group per workgroup
+        }
+    }
     if (fast && kStageable && tg <= (G == 64 ? 64 : 128))
         hipLaunchKernelGGL((pack128_kernel<T, G, false, kStageable>), grid, dim3(kWave * pack128_waves<G>()), 0,
                            stream, keys, head_stride, tokens, tg, ks, km, kl, kd, cap, off, AppendArgs<T>{});
