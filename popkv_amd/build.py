@@ -19,7 +19,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB_DIR = PKG / "_lib"
 LIB_PATH = LIB_DIR / "libpopkv_hip.so"
-SOURCES = ("pack.hip", "score.hip", "select.hip", "attention.hip", "capi.hip")
+SOURCES = ("pack.hip", "score.hip", "select.hip", "attention.hip", "dense.hip", "capi.hip")
 ARCH = os.environ.get("POPKV_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

@@ -27,6 +27,7 @@
 // launch is far cheaper.)
 #include <type_traits>
 
+#include "attention_common.h"
 #include "device_common.h"
 #include "pack128.h"
 #include "kernels.h"
@@ -36,8 +37,6 @@
 namespace popkv {
 namespace {
 
-constexpr int kAttnThreads = 256;
-constexpr int kAttnWaves = kAttnThreads / kWave;
 constexpr int kAttnStage = 1024;  // indices of one split staged in LDS
 // Polls of the single-launch layer step's select blocks before they give up
 // waiting for the scorer (each poll is a device-coherent load round trip and
@@ -51,107 +50,6 @@ __device__ __forceinline__ void load_row8(const T* p, int dim0, int d, float v[8
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = 0.0f;
-    }
-}
-
-struct SoftmaxState {
-    float m, l, acc[8];
-};
-
-__device__ __forceinline__ void merge_state(SoftmaxState& a, float m2, float l2, const float* acc2) {
-    const float mm = fmaxf(a.m, m2);
-    if (mm == -INFINITY) return;
-    const float wa = a.m == -INFINITY ? 0.0f : __expf(a.m - mm);
-    const float wb = m2 == -INFINITY ? 0.0f : __expf(m2 - mm);
-    a.l = a.l * wa + l2 * wb;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a.acc[i] = a.acc[i] * wa + acc2[i] * wb;
-    a.m = mm;
-}
-
-// Writes a workgroup's (m, l, acc[d]) to dst: the row slots of each wave
-// (lanes with equal dim slice) merge through shuffles, the waves through LDS.
-// All threads of the block call it.
-// Partial states handed from one workgroup to another inside a kernel (the
-// layer step's fused merge) are written and read as device-scope relaxed
-// atomics: plain global stores / loads with the device-coherence bit, which
-// go through to memory instead of staying in one XCD's L2, so no L2
-// write-back or invalidate is needed for them.
-// The fused merges hand chunk states from workgroup to workgroup with no
-// release/acquire pair: the states are stored with relaxed agent-scope
-// atomic stores, each wave then waits with "s_waitcnt vmcnt(0)", the block
-// meets at a barrier, and one relaxed agent-scope atomic add takes the
-// ticket; the last block reads the states with relaxed agent-scope atomic
-// loads.  That is correct on gfx942 / gfx950 because (1) an agent-scope
-// atomic store or load is a global store / load with the sc1 bit, which
-// writes through and reads past the XCD's non-coherent L2 to the device's
-// coherence point, and (2) stores count in vmcnt on these targets, so
-// vmcnt(0) returns only once every store of the wave is acknowledged by
-// that point -- before the ticket is taken.  On targets that count stores
-// in a separate vscnt (gfx10 and later) or that cache agent-scope stores,
-// the wait would not cover the states: the build refuses them.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__) && !defined(__gfx942__)
-#error "the fused merge's hand-off relies on gfx942/gfx950 store acknowledgement (vmcnt) and sc1 write-through"
-#endif
-
-template <bool COH>
-__device__ __forceinline__ void st_f32(float* p, float v) {
-    if constexpr (COH) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else *p = v;
-}
-template <bool COH>
-__device__ __forceinline__ float ld_f32(const float* p) {
-    if constexpr (COH) return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else return *p;
-}
-
-template <int LPR>
-__device__ __forceinline__ void store_partial(SoftmaxState st, int lane, int wave, int dim0, int d, float* dst,
-                                              bool coherent = false) {
-    auto merge_xor = [&](auto mtag) {
-        constexpr int M = decltype(mtag)::value;
-        const float m2 = lane_xor<M>(st.m);
-        const float l2 = lane_xor<M>(st.l);
-        float a2[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) a2[i] = lane_xor<M>(st.acc[i]);
-        merge_state(st, m2, l2, a2);
-    };
-    if constexpr (LPR <= 8) merge_xor(std::integral_constant<int, 8>{});
-    if constexpr (LPR <= 16) merge_xor(std::integral_constant<int, 16>{});
-    merge_xor(std::integral_constant<int, 32>{});
-    __shared__ float s_m[kAttnWaves], s_l[kAttnWaves];
-    __shared__ float s_acc[kAttnWaves][256];
-    if (lane < LPR) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s_acc[wave][dim0 + i] = st.acc[i];
-        if (lane == 0) { s_m[wave] = st.m; s_l[wave] = st.l; }
-    }
-    __syncthreads();
-    const int dim = threadIdx.x;
-    float mx = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) mx = fmaxf(mx, s_m[w]);
-    float l = 0.0f, a = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) {
-        if (s_m[w] == -INFINITY) continue;
-        const float wt = __expf(s_m[w] - mx);
-        l += s_l[w] * wt;
-        if (dim < d) a += s_acc[w][dim] * wt;
-    }
-    if (coherent) {
-        if (dim < d) st_f32<true>(dst + 2 + dim, a);
-        if (dim == 0) {
-            st_f32<true>(dst, mx);
-            st_f32<true>(dst + 1, l);
-        }
-    } else {
-        if (dim < d) dst[2 + dim] = a;
-        if (dim == 0) {
-            dst[0] = mx;
-            dst[1] = l;
-        }
     }
 }
 
@@ -395,119 +293,6 @@ __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(const float* 
 }
 
 
-// Split states a merge loads in its first burst (and per batch after it).
-constexpr int kMergeFirst = 16;
-
-// Row of current_k / current_v for merge block h, and (for a batched step)
-// the row's current-token index and its slot k in the indices: sequence b =
-// h / q_heads has min(tokens[b], bound) cached tokens (*current holds the
-// launch bound on entry).  Unbatched: KV head head_to_kv[h] (clamped), or
-// h / (QH / KVH) without a mapping (the dense layers).
-__device__ __forceinline__ int64_t merge_kv_row(const SeqTable& seq, const int64_t* __restrict__ head_to_kv, int h,
-                                                int kv_heads, int rows, int64_t* idx_slot, int64_t* current) {
-    if (seq.tokens != nullptr) {
-        const int64_t b = h / seq.q_heads;
-        const int64_t raw = seq.tokens[b];
-        if (seq.status != nullptr && (raw < 0 || raw > *current) && (threadIdx.x & (kWave - 1)) == 0)
-            atomicOr(seq.status, 2);
-        *current = seq_tokens_of(seq, b, *current);
-        *idx_slot = min(static_cast<int64_t>(seq.budget) - 1, *current);
-        return b * seq.kv_heads +
-               min(max(head_to_kv[h - b * seq.q_heads], static_cast<int64_t>(0)), static_cast<int64_t>(seq.kv_heads - 1));
-    }
-    return head_to_kv != nullptr ? min(max(head_to_kv[h], static_cast<int64_t>(0)), static_cast<int64_t>(kv_heads - 1))
-                                 : h / (rows / kv_heads);
-}
-
-// Merge of one head by one wave (lane l owning dims l and l + 64): the
-// head's nsplit states ps[s] = (m, l, acc[128]) plus the current token
-// (logit qh . ck * scale, value cv), written to outh in the query dtype.
-// No LDS or barrier: the split maxima and denominators are wave reductions
-// (lane s holds split s of each 64-split group), and the weights reach the
-// accumulation through readlane.  qh, ck, cv, the first group's maxima and
-// denominators and the first NF splits' accumulators are loaded in one
-// burst, so a layer step's merge pays one memory latency for all of them;
-// further splits follow in batches of NF.  Accumulation
-// order: the current token, then the splits in ascending order.  COH: the
-// states are read with device-coherent loads (written by other workgroups
-// of the same kernel).
-template <typename T, bool COH, int NF = kMergeFirst>
-__device__ __forceinline__ void merge_head(const float* __restrict__ ps, int nsplit, const T* __restrict__ qh,
-                                           const T* __restrict__ ck, const T* __restrict__ cv, float scale,
-                                           T* __restrict__ outh) {
-    constexpr int S = 128 + 2;
-    const int lane = threadIdx.x & (kWave - 1);
-    // the burst (with nsplit == 0 the accumulator loads read split 0's slot,
-    // which every workspace holds, and are not used)
-    const float q0 = Elem<T>::load(qh, lane), q1 = Elem<T>::load(qh, lane + 64);
-    const float k0 = Elem<T>::load(ck, lane), k1 = Elem<T>::load(ck, lane + 64);
-    const float v0 = Elem<T>::load(cv, lane), v1 = Elem<T>::load(cv, lane + 64);
-    float m0 = -INFINITY, l0 = 0.0f;  // split `lane`
-    if (lane < nsplit) {
-        m0 = ld_f32<COH>(ps + (static_cast<int64_t>(lane) * S));
-        l0 = ld_f32<COH>(ps + (static_cast<int64_t>(lane) * S + 1));
-    }
-    const int nf = min(nsplit, NF);
-    float a0[NF], a1[NF];
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-        const int64_t so = static_cast<int64_t>(max(min(j, nf - 1), 0)) * S + 2;
-        a0[j] = ld_f32<COH>(ps + (so + lane));
-        a1[j] = ld_f32<COH>(ps + (so + lane + 64));
-    }
-    // the maxima of every split and the current token's logit
-    float mx = m0;
-    for (int s0 = kWave; s0 < nsplit; s0 += kWave)
-        if (s0 + lane < nsplit) mx = fmaxf(mx, ld_f32<COH>(ps + (static_cast<int64_t>(s0 + lane) * S)));
-    const float cur_m = wave_sum(q0 * k0 + q1 * k1) * scale;
-    mx = fmaxf(wave_max(mx), cur_m);
-    const float wc = __expf(cur_m - mx);
-    const float w0 = m0 == -INFINITY ? 0.0f : __expf(m0 - mx);
-    float den = l0 * w0, num0 = wc * v0, num1 = wc * v1;
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-        if (j < nf) {
-            const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w0), j));
-            num0 = fmaf(ws, a0[j], num0);
-            num1 = fmaf(ws, a1[j], num1);
-        }
-    }
-    for (int s0 = 0; s0 < nsplit; s0 += kWave) {
-        float w = w0;
-        if (s0 > 0) {
-            float m = -INFINITY, l = 0.0f;
-            if (s0 + lane < nsplit) {
-                m = ld_f32<COH>(ps + (static_cast<int64_t>(s0 + lane) * S));
-                l = ld_f32<COH>(ps + (static_cast<int64_t>(s0 + lane) * S + 1));
-            }
-            w = m == -INFINITY ? 0.0f : __expf(m - mx);
-            den += l * w;
-        }
-        const int n = min(kWave, nsplit - s0);
-        for (int b = s0 == 0 ? nf : 0; b < n; b += NF) {
-            float c0[NF], c1[NF];
-#pragma unroll
-            for (int j = 0; j < NF; ++j) {
-                const int64_t so = static_cast<int64_t>(s0 + min(b + j, n - 1)) * S + 2;
-                c0[j] = ld_f32<COH>(ps + (so + lane));
-                c1[j] = ld_f32<COH>(ps + (so + lane + 64));
-            }
-#pragma unroll
-            for (int j = 0; j < NF; ++j) {
-                if (b + j < n) {
-                    const float ws =
-                        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), b + j));
-                    num0 = fmaf(ws, c0[j], num0);
-                    num1 = fmaf(ws, c1[j], num1);
-                }
-            }
-        }
-    }
-    den = wave_sum(den) + wc;
-    Elem<T>::store(outh, lane, num0 / den);
-    Elem<T>::store(outh, lane + 64, num1 / den);
-}
-
 // ---------------------------------------------------------------- layer step
 
 // Layer-step attention.  Row slot q of a workgroup (16 lanes, one 16-byte
@@ -516,72 +301,6 @@ __device__ __forceinline__ void merge_head(const float* __restrict__ ps, int nsp
 // contiguous (token stride = head_dim = 128).  For 16-bit types the Q.K
 // products use v_dot2 (two products accumulated in fp32 per instruction).
 constexpr int kSplitRows = 256;  // the reference's split: selected tokens per workgroup
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
-// Dot product of 8 packed 16-bit elements with v_dot2 (fp32 accumulation).
-template <typename T>
-__device__ __forceinline__ float dot8(const uint4& a, const uint4& b) {
-    auto d2 = [](uint32_t x, uint32_t y, float c) {
-        if constexpr (Elem<T>::kDtype == POPKV_DTYPE_BF16)
-            return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x), __builtin_bit_cast(bf16x2_t, y), c,
-                                                   false);
-        else
-            return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, x), __builtin_bit_cast(f16x2_t, y), c, false);
-    };
-    return d2(a.w, b.w, d2(a.z, b.z, d2(a.y, b.y, d2(a.x, b.x, 0.0f))));
-}
-
-__device__ __forceinline__ void init_state(SoftmaxState& st) {
-    st.m = -INFINITY;
-    st.l = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) st.acc[i] = 0.0f;
-}
-
-// Folds NB gathered rows (this lane's 8-element slices of K and V; the 16
-// lanes of a row slot hold one row) into the lane's online-softmax state.
-// Rows with live[b] false get weight exactly 0.
-template <typename T, int NB>
-__device__ __forceinline__ void fold_rows(SoftmaxState& st, const Raw8<T>& qr, const Raw8<T> (&kr)[NB],
-                                          const Raw8<T> (&vr)[NB], const bool (&live)[NB], float scale) {
-    float logit[NB];
-    float bm = -INFINITY;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        float dot;
-        if constexpr (sizeof(T) == 2) {
-            dot = dot8<T>(qr.u, kr[b].u);
-        } else {
-            dot = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dot = fmaf(qr.get(i), kr[b].get(i), dot);
-        }
-        dot = row_sum<16>(dot);
-        logit[b] = live[b] ? dot * scale : -INFINITY;
-        bm = fmaxf(bm, logit[b]);
-    }
-    // The compiler sinks the V loads into this branch, so a batch's V rows
-    // are requested only once its K rows have arrived.  A branch-free form
-    // with every K and V request in flight at once measured slower on the
-    // layer step's gathers (C1 select + attention kernel 18.6 vs 17.1 us).
-    const float mnew = fmaxf(st.m, bm);
-    if (mnew != -INFINITY) {
-        const float alpha = __expf(st.m - mnew);  // st.m = -inf gives 0
-        st.l *= alpha;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) st.acc[i] *= alpha;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const float p = __expf(logit[b] - mnew);  // -inf logit gives 0
-            st.l += p;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) st.acc[i] = fmaf(p, vr[b].get(i), st.acc[i]);
-        }
-        st.m = mnew;
-    }
-}
 
 // Block -> (chunk, head) of the layer step's select + attention grid
 // (nchunks * QH blocks).  With kv_groups (KV heads a multiple of 8, query
@@ -1261,348 +980,6 @@ __global__ __launch_bounds__(kScoreThreads) void layer_step_fused_kernel(
         StepAppendArgs<T>{}, win, id - static_cast<uint32_t>(nscore));
 }
 
-// Dense attention (the reference's full layers, popkv.py:1022-1038): every
-// prefix token attends; the current token joins in the merge, as in the
-// layer step.  Splits of kDenseSplit tokens.
-constexpr int kDenseSplit = 512;
-// The MFMA kernel fuses the merge for up to this many splits (64 x 512 =
-// 32768 tokens: the merge loads every split's accumulators in one burst);
-// longer prefixes take the separate wide merge.
-constexpr int kDenseFusedMaxSplits = 64;
-
-// Dense attention, one GQA group per workgroup: the QPK query heads of KV
-// head g share every K/V row, so workgroup (s, g) reads each row of its
-// 512-token split once and folds it into QPK online-softmax states (one Q.K
-// dot and one V update per head per row).  Memory traffic is one pass over
-// the KV head's rows instead of QPK.
-template <typename T, int NB, int QPK>
-__global__ __launch_bounds__(kAttnThreads) void attn_dense_gqa_kernel(
-    const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, int64_t k_hs, int64_t v_hs,
-    int64_t tokens, float scale, float* __restrict__ partials, int nsplit) {
-    constexpr int D = 128, LPR = 16, SLOTS = kWave / LPR, ROWS_PER_PASS = SLOTS * kAttnWaves;
-    const int g = blockIdx.y;
-    const int s = blockIdx.x;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int slot = wave * SLOTS + lane / LPR;
-    const int dim0 = (lane % LPR) * 8;
-    Raw8<T> qr[QPK];
-#pragma unroll
-    for (int j = 0; j < QPK; ++j) qr[j].load(q + static_cast<int64_t>(g * QPK + j) * D + dim0);
-    const int t0 = s * kDenseSplit;
-    const int n_rows = static_cast<int>(min<int64_t>(kDenseSplit, tokens - t0));
-    const char* kb = reinterpret_cast<const char*>(kc + g * k_hs) + dim0 * sizeof(T);
-    const char* vb = reinterpret_cast<const char*>(vc + g * v_hs) + dim0 * sizeof(T);
-    SoftmaxState st[QPK];
-#pragma unroll
-    for (int j = 0; j < QPK; ++j) init_state(st[j]);
-    for (int base = 0; base < n_rows; base += ROWS_PER_PASS * NB) {
-        Raw8<T> kr[NB], vr[NB];
-        bool live[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int r = base + b * ROWS_PER_PASS + slot;
-            live[b] = r < n_rows;
-            const uint32_t off = static_cast<uint32_t>(t0 + (live[b] ? r : 0)) * (D * sizeof(T));
-            kr[b].load(reinterpret_cast<const T*>(kb + off));
-            vr[b].load(reinterpret_cast<const T*>(vb + off));
-        }
-#pragma unroll
-        for (int j = 0; j < QPK; ++j) fold_rows<T, NB>(st[j], qr[j], kr, vr, live, scale);
-    }
-#pragma unroll
-    for (int j = 0; j < QPK; ++j) {
-        store_partial<LPR>(st[j], lane, wave, dim0, D,
-                           partials + (static_cast<int64_t>(g * QPK + j) * nsplit + s) * (D + 2));
-        __syncthreads();  // store_partial's LDS is reused by the next head
-    }
-}
-
-// Dense attention for GQA groups of four query heads in 16-bit types, with
-// Q.K on the matrix cores: per 16-token tile one v_mfma_f32_16x16x32 chain
-// (4 steps of 32 dims) multiplies A = the group's query rows (rows 0-3; rows
-// 4-15 zero) by B = the tile's K rows (column n = token n), so lanes 0-15
-// end with the four heads' logits of token `lane` (C layout: lane l holds
-// rows 4*(l/16) .. +3 of column l % 16; A and B: lane l holds k-elements
-// 8*(l/16) .. +7 of row / column l % 16).  The tile's softmax runs on those
-// lanes (DPP row maxima, one running max per head and wave), the weights go
-// through LDS to the four 16-lane row slots, and each slot folds 4 of the
-// tile's V rows into its accumulators (8 dims per lane) with the VALU.
-// Workgroup (split, KV head) = 4 waves of 128 tokens; tiles double-buffered
-// (the next tile's K and V loads issued before the current tile is folded).
-template <typename T> struct MfmaVec8;
-template <> struct MfmaVec8<bf16_t> { typedef __bf16 type __attribute__((ext_vector_type(8))); };
-template <> struct MfmaVec8<f16_t> { typedef _Float16 type __attribute__((ext_vector_type(8))); };
-typedef float mfma_f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-__device__ __forceinline__ mfma_f32x4 mfma_16x16x32(uint4 a, uint4 b, mfma_f32x4 c) {
-    using V = typename MfmaVec8<T>::type;
-    if constexpr (std::is_same_v<T, bf16_t>)
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(V, a), __builtin_bit_cast(V, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(V, a), __builtin_bit_cast(V, b), c, 0, 0, 0);
-}
-
-template <typename T>
-__global__ __launch_bounds__(kAttnThreads) void attn_dense_mfma_kernel(
-    const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, int64_t k_hs, int64_t v_hs,
-    int64_t tokens, float scale, float* __restrict__ partials, int nsplit, uint32_t* __restrict__ tickets,
-    const T* __restrict__ cur_k, const T* __restrict__ cur_v, T* __restrict__ out) {
-    constexpr int D = 128, QPK = 4, TILE = 16;
-    constexpr int WTOK = kDenseSplit / kAttnWaves;  // tokens per wave
-    constexpr int NT = WTOK / TILE;                  // tiles per wave
-    const int g = blockIdx.y;
-    const int s = blockIdx.x;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int col = lane & 15;  // MFMA row / column; the V dim slice 8*col
-    const int grp = lane >> 4;  // MFMA k-group; the V row slot
-    const int t0 = s * kDenseSplit;
-    const int n_rows = static_cast<int>(min<int64_t>(kDenseSplit, tokens - t0));
-    const int w0 = wave * WTOK;
-    uint4 qa[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        qa[i] = col < QPK ? *reinterpret_cast<const uint4*>(q + static_cast<int64_t>(g * QPK + col) * D + 32 * i + 8 * grp)
-                          : make_uint4(0u, 0u, 0u, 0u);
-    const char* kb = reinterpret_cast<const char*>(kc + g * k_hs) + 8 * grp * sizeof(T);
-    const char* vb = reinterpret_cast<const char*>(vc + g * v_hs) + 8 * col * sizeof(T);
-    // rows past the split's end re-read the split's first row (weight 0)
-    auto load_tile = [&](int it, uint4 (&kt)[4], uint4 (&vt)[4]) {
-        const int rk = w0 + it * TILE + col;
-        const uint32_t ko = static_cast<uint32_t>(t0 + (rk < n_rows ? rk : 0)) * (D * sizeof(T));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) kt[i] = *reinterpret_cast<const uint4*>(kb + ko + 32 * i * sizeof(T));
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int rv = w0 + it * TILE + 4 * grp + r;
-            const uint32_t vo = static_cast<uint32_t>(t0 + (rv < n_rows ? rv : 0)) * (D * sizeof(T));
-            vt[r] = *reinterpret_cast<const uint4*>(vb + vo);
-        }
-    };
-    __shared__ float4 s_p[kAttnWaves][TILE];
-    float m_run[QPK], lsum[QPK], acc[QPK][8];
-#pragma unroll
-    for (int j = 0; j < QPK; ++j) {
-        m_run[j] = -INFINITY;
-        lsum[j] = 0.0f;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) acc[j][d] = 0.0f;
-    }
-    auto fold_tile = [&](int it, const uint4 (&kt)[4], const uint4 (&vt)[4]) {
-        mfma_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) c = mfma_16x16x32<T>(qa[i], kt[i], c);
-        const bool live = w0 + it * TILE + col < n_rows;
-        float p[QPK], alpha[QPK];
-        bool rescale = false;
-#pragma unroll
-        for (int j = 0; j < QPK; ++j) {
-            const float sj = live ? c[j] * scale : -INFINITY;
-            float mx = fmaxf(sj, dpp_mov<0xB1>(sj));
-            mx = fmaxf(mx, dpp_mov<0x4E>(mx));
-            mx = fmaxf(mx, dpp_mov<0x141>(mx));
-            mx = fmaxf(mx, dpp_mov<0x140>(mx));
-            const float mt = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mx), 0));
-            const float mn = fmaxf(m_run[j], mt);
-            alpha[j] = mn == -INFINITY ? 1.0f : __expf(m_run[j] - mn);  // m_run = -inf gives 0
-            p[j] = mn == -INFINITY ? 0.0f : __expf(sj - mn);           // dead rows give 0
-            rescale = rescale || mn != m_run[j];
-            m_run[j] = mn;
-        }
-        if (lane < TILE) s_p[wave][col] = make_float4(p[0], p[1], p[2], p[3]);
-        // the wave reads its own weights next: one wave's LDS operations complete in order
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (rescale) {  // wave-uniform: some head's running max moved
-#pragma unroll
-            for (int j = 0; j < QPK; ++j) {
-                lsum[j] *= alpha[j];
-#pragma unroll
-                for (int d = 0; d < 8; ++d) acc[j][d] *= alpha[j];
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float4 pr = s_p[wave][4 * grp + r];
-            Raw8<T> v;
-            v.u = vt[r];
-            float vf[8];
-#pragma unroll
-            for (int d = 0; d < 8; ++d) vf[d] = v.get(d);
-            const float pj[QPK] = {pr.x, pr.y, pr.z, pr.w};
-#pragma unroll
-            for (int j = 0; j < QPK; ++j) {
-                lsum[j] += pj[j];
-#pragma unroll
-                for (int d = 0; d < 8; ++d) acc[j][d] = fmaf(pj[j], vf[d], acc[j][d]);
-            }
-        }
-        // the next tile's weights overwrite s_p[wave] only after every lane has read
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    // a ring of AHEAD + 1 tiles: tile it + AHEAD is issued before tile it is
-    // folded (fully unrolled, so every ring index is a constant)
-    constexpr int AHEAD = 1;
-    uint4 kt[AHEAD + 1][4], vt[AHEAD + 1][4];
-#pragma unroll
-    for (int it = 0; it < AHEAD; ++it) load_tile(it, kt[it], vt[it]);
-#pragma unroll
-    for (int it = 0; it < NT; ++it) {
-        if (it + AHEAD < NT) load_tile(it + AHEAD, kt[(it + AHEAD) % (AHEAD + 1)], vt[(it + AHEAD) % (AHEAD + 1)]);
-        fold_tile(it, kt[it % (AHEAD + 1)], vt[it % (AHEAD + 1)]);
-    }
-    const bool fused = tickets != nullptr;  // the merge runs in the group's last block (below)
-#pragma unroll
-    for (int j = 0; j < QPK; ++j) {
-        SoftmaxState st;
-        st.m = m_run[j];
-        st.l = lsum[j];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) st.acc[d] = acc[j][d];
-        store_partial<16>(st, lane, wave, 8 * col, D,
-                          partials + (static_cast<int64_t>(g * QPK + j) * nsplit + s) * (D + 2), fused);
-        __syncthreads();  // store_partial's LDS is reused by the next head
-    }
-    if (!fused) return;
-    // Fused merge, as in the layer step's select + attention kernel: the
-    // states went out with device-coherent stores; once this block's are
-    // acknowledged (the gfx942 / gfx950 rule stated at st_f32) it takes a
-    // ticket on tickets[g] (zero between calls), and the group's last block
-    // merges each of its heads' splits with the current token (wave j: head
-    // g * QPK + j, every split's accumulators loaded in one burst of up to
-    // 64) and resets the ticket.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    __shared__ uint32_t s_last;
-    if (threadIdx.x == 0) {
-        const uint32_t old = __hip_atomic_fetch_add(&tickets[g], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = old + 1u == static_cast<uint32_t>(nsplit) ? 1u : 0u;
-    }
-    __syncthreads();
-    if (s_last == 0u) return;
-    if (threadIdx.x == 0) __hip_atomic_store(&tickets[g], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int h = g * QPK + wave;
-    merge_head<T, true, 64>(partials + static_cast<int64_t>(h) * nsplit * (D + 2), nsplit,
-                            q + static_cast<int64_t>(h) * D, cur_k + static_cast<int64_t>(g) * D,
-                            cur_v + static_cast<int64_t>(g) * D, scale, out + static_cast<int64_t>(h) * D);
-}
-
-
-// Layer-step merge kernel (the unfused form: popkv_layer_step_attention's
-// timing runs, and the dense layers): one wave per head, see merge_head.
-template <typename T>
-__global__ __launch_bounds__(kWave) void attn_merge_current_kernel(
-    const float* __restrict__ partials, int nsplit, const T* __restrict__ q, const T* __restrict__ cur_k,
-    const T* __restrict__ cur_v, const int64_t* __restrict__ head_to_kv, int kv_heads, float scale,
-    T* __restrict__ out, int64_t* __restrict__ idx_out, int64_t idx_stride, int64_t idx_slot, int64_t current,
-    SeqTable seq) {
-    constexpr int D = 128, S = D + 2;
-    const int h = blockIdx.x;
-    const int lane = threadIdx.x;
-    // the current token's index slot of the layer step's int64 indices, and
-    // the KV row of its current k/v (no mapping: the plain GQA grouping of
-    // the dense layers)
-    const int64_t kvh = merge_kv_row(seq, head_to_kv, h, kv_heads, gridDim.x, &idx_slot, &current);
-    if (idx_out != nullptr && lane == 0) idx_out[static_cast<int64_t>(h) * idx_stride + idx_slot] = current;
-    merge_head<T, false>(partials + static_cast<int64_t>(h) * nsplit * S, nsplit, q + static_cast<int64_t>(h) * D,
-                         cur_k + kvh * D, cur_v + kvh * D, scale, out + static_cast<int64_t>(h) * D);
-}
-
-// Merge for many splits (dense layers: one split per 512 tokens): four
-// waves per head, wave w folding splits [16w, 16w + 16), [64 + 16w, ...) --
-// each batch of 16 in one load burst -- into a running (m, l, acc) state;
-// wave 0 then combines the four states with the current token.  The layer
-// step's merge (at most 16 splits at C1) keeps the one-wave kernel above.
-constexpr int kMergeWaves = 4;
-
-template <typename T>
-__global__ __launch_bounds__(kWave * kMergeWaves) void attn_merge_wide_kernel(
-    const float* __restrict__ partials, int nsplit, const T* __restrict__ q, const T* __restrict__ cur_k,
-    const T* __restrict__ cur_v, const int64_t* __restrict__ head_to_kv, int kv_heads, float scale,
-    T* __restrict__ out, int64_t* __restrict__ idx_out, int64_t idx_stride, int64_t idx_slot, int64_t current,
-    SeqTable seq) {
-    constexpr int D = 128, S = D + 2;
-    const int h = blockIdx.x;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int64_t kvh = merge_kv_row(seq, head_to_kv, h, kv_heads, gridDim.x, &idx_slot, &current);
-    if (idx_out != nullptr && threadIdx.x == 0) idx_out[static_cast<int64_t>(h) * idx_stride + idx_slot] = current;
-    const float* ps = partials + static_cast<int64_t>(h) * nsplit * S;
-    float q0 = 0.0f, q1 = 0.0f, k0 = 0.0f, k1 = 0.0f, v0 = 0.0f, v1 = 0.0f;
-    if (wave == 0) {  // the current token's operands, in flight during the splits
-        const T* qh = q + static_cast<int64_t>(h) * D;
-        q0 = Elem<T>::load(qh, lane);
-        q1 = Elem<T>::load(qh, lane + 64);
-        k0 = Elem<T>::load(cur_k + kvh * D, lane);
-        k1 = Elem<T>::load(cur_k + kvh * D, lane + 64);
-        v0 = Elem<T>::load(cur_v + kvh * D, lane);
-        v1 = Elem<T>::load(cur_v + kvh * D, lane + 64);
-    }
-    float wm = -INFINITY, wl = 0.0f, a0 = 0.0f, a1 = 0.0f;
-    for (int s0 = wave * kMergeFirst; s0 < nsplit; s0 += kMergeWaves * kMergeFirst) {
-        const int nb = min(kMergeFirst, nsplit - s0);
-        float m = -INFINITY, l = 0.0f;
-        if (lane < nb) {
-            m = ps[static_cast<int64_t>(s0 + lane) * S];
-            l = ps[static_cast<int64_t>(s0 + lane) * S + 1];
-        }
-        float c0[kMergeFirst], c1[kMergeFirst];
-#pragma unroll
-        for (int j = 0; j < kMergeFirst; ++j) {
-            const int64_t so = static_cast<int64_t>(s0 + min(j, nb - 1)) * S + 2;
-            c0[j] = ps[so + lane];
-            c1[j] = ps[so + lane + 64];
-        }
-        const float nm = fmaxf(wm, wave_max(m));
-        const float alpha = wm == -INFINITY ? 0.0f : __expf(wm - nm);
-        const float w = m == -INFINITY ? 0.0f : __expf(m - nm);
-        wl = wl * alpha + wave_sum(l * w);
-        a0 *= alpha;
-        a1 *= alpha;
-#pragma unroll
-        for (int j = 0; j < kMergeFirst; ++j) {
-            if (j < nb) {
-                const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), j));
-                a0 = fmaf(ws, c0[j], a0);
-                a1 = fmaf(ws, c1[j], a1);
-            }
-        }
-        wm = nm;
-    }
-    __shared__ float s_m[kMergeWaves], s_l[kMergeWaves], s_a[kMergeWaves][D];
-    if (lane == 0) {
-        s_m[wave] = wm;
-        s_l[wave] = wl;
-    }
-    s_a[wave][lane] = a0;
-    s_a[wave][lane + 64] = a1;
-    __syncthreads();
-    if (wave == 0) {
-        const float cur_m = wave_sum(q0 * k0 + q1 * k1) * scale;
-        float mx = cur_m;
-#pragma unroll
-        for (int w = 0; w < kMergeWaves; ++w) mx = fmaxf(mx, s_m[w]);
-        const float wc = __expf(cur_m - mx);
-        float den = wc, num0 = wc * v0, num1 = wc * v1;
-#pragma unroll
-        for (int w = 0; w < kMergeWaves; ++w) {
-            if (s_m[w] != -INFINITY) {
-                const float f = __expf(s_m[w] - mx);
-                den += s_l[w] * f;
-                num0 = fmaf(f, s_a[w][lane], num0);
-                num1 = fmaf(f, s_a[w][lane + 64], num1);
-            }
-        }
-        Elem<T>::store(out + static_cast<int64_t>(h) * D, lane, num0 / den);
-        Elem<T>::store(out + static_cast<int64_t>(h) * D, lane + 64, num1 / den);
-    }
-}
-
 // API-path partial attention, fast form (head_dim 128, contiguous K/V rows,
 // the reference's 256-row splits, 16-byte aligned index rows): row slot q
 // owns the split's entries [16q, 16q + 16) and reads them with 16-byte
@@ -1913,24 +1290,6 @@ hipError_t launch_select_chunks_t(const void* q, const void* kc, const void* vc,
 }
 
 template <typename T>
-hipError_t launch_merge_current_t(const float* partials, int nsplit, const void* q, const void* cur_k,
-                                  const void* cur_v, const int64_t* h2k, int q_heads, int kv_heads, void* out,
-                                  int64_t* idx_out, int64_t idx_stride, int64_t idx_slot, int64_t current,
-                                  const SeqTable& seq, hipStream_t stream) {
-    const float scale = static_cast<float>(1.0 / sqrt(128.0));
-    if (nsplit > kMergeFirst)
-        hipLaunchKernelGGL((attn_merge_wide_kernel<T>), dim3(static_cast<unsigned>(q_heads)),
-                           dim3(kWave * kMergeWaves), 0, stream, partials, nsplit, static_cast<const T*>(q),
-                           static_cast<const T*>(cur_k), static_cast<const T*>(cur_v), h2k, kv_heads, scale,
-                           static_cast<T*>(out), idx_out, idx_stride, idx_slot, current, seq);
-    else
-        hipLaunchKernelGGL((attn_merge_current_kernel<T>), dim3(static_cast<unsigned>(q_heads)), dim3(kWave), 0,
-                           stream, partials, nsplit, static_cast<const T*>(q), static_cast<const T*>(cur_k),
-                           static_cast<const T*>(cur_v), h2k, kv_heads, scale, static_cast<T*>(out), idx_out,
-                           idx_stride, idx_slot, current, seq);
-    return hipGetLastError();
-}
-template <typename T>
 hipError_t launch_layer_step_fused_t(const void* queries, const int32_t* k_sign, const int32_t* k_mag,
                                      const uint16_t* k_low, const uint16_t* k_delta, int64_t capacity,
                                      const void* prefix_k, const void* prefix_v, int64_t k_hs, int64_t v_hs,
@@ -2052,81 +1411,4 @@ hipError_t launch_attention_select_chunks(const void* queries, int dtype, const 
     }
 }
 
-hipError_t launch_merge_current(const float* partials, int nsplit, const void* queries, int dtype,
-                                const void* current_k, const void* current_v, const int64_t* head_to_kv, int q_heads,
-                                int kv_heads, void* output, int64_t* idx_out, int64_t idx_stride, int64_t idx_slot,
-                                int64_t current, const SeqTable& seq, hipStream_t stream) {
-    switch (dtype) {
-        case POPKV_DTYPE_F32:
-            return launch_merge_current_t<float>(partials, nsplit, queries, current_k, current_v, head_to_kv, q_heads,
-                                                 kv_heads, output, idx_out, idx_stride, idx_slot, current, seq,
-                                                 stream);
-        case POPKV_DTYPE_F16:
-            return launch_merge_current_t<f16_t>(partials, nsplit, queries, current_k, current_v, head_to_kv, q_heads,
-                                                 kv_heads, output, idx_out, idx_stride, idx_slot, current, seq,
-                                                 stream);
-        default:
-            return launch_merge_current_t<bf16_t>(partials, nsplit, queries, current_k, current_v, head_to_kv,
-                                                  q_heads, kv_heads, output, idx_out, idx_stride, idx_slot, current,
-                                                  seq, stream);
-    }
-}
-
-
-namespace {
-template <typename T>
-hipError_t launch_dense_t(const void* q, const void* kc, const void* vc, int64_t k_hs, int64_t v_hs, int64_t tokens,
-                          int nsplit, int q_heads, int kv_heads, float* partials, const DenseMerge* merge,
-                          hipStream_t stream) {
-    const float scale = static_cast<float>(1.0 / sqrt(128.0));
-    const dim3 grid(static_cast<unsigned>(nsplit), static_cast<unsigned>(kv_heads));
-    const T *q_ = static_cast<const T*>(q), *k_ = static_cast<const T*>(kc), *v_ = static_cast<const T*>(vc);
-#define POPKV_DENSE(NB, QPK)                                                                                   \
-    hipLaunchKernelGGL((attn_dense_gqa_kernel<T, NB, QPK>), grid, dim3(kAttnThreads), 0, stream, q_, k_, v_, k_hs, \
-                       v_hs, tokens, scale, partials, nsplit)
-    if constexpr (sizeof(T) == 2) {
-        if (q_heads == 4 * kv_heads) {
-            const bool fuse = merge != nullptr && nsplit <= kDenseFusedMaxSplits;
-            hipLaunchKernelGGL((attn_dense_mfma_kernel<T>), grid, dim3(kAttnThreads), 0, stream, q_, k_, v_, k_hs, v_hs,
-                               tokens, scale, partials, nsplit, fuse ? merge->tickets : nullptr,
-                               fuse ? static_cast<const T*>(merge->current_k) : nullptr,
-                               fuse ? static_cast<const T*>(merge->current_v) : nullptr,
-                               fuse ? static_cast<T*>(merge->output) : nullptr);
-            return hipGetLastError();
-        }
-    }
-    switch (q_heads / kv_heads) {
-        case 1: POPKV_DENSE((sizeof(T) == 4 ? 8 : 16), 1); break;
-        case 2: POPKV_DENSE(8, 2); break;
-        case 4: POPKV_DENSE(4, 4); break;  // 127 VGPRs; 8 rows: 180 (measured 0.3 us slower)
-        default: POPKV_DENSE(4, 8); break;
-    }
-#undef POPKV_DENSE
-    return hipGetLastError();
-}
-}  // namespace
-
-int dense_splits(int64_t tokens) { return static_cast<int>((tokens + kDenseSplit - 1) / kDenseSplit); }
-
-bool dense_merge_fuses(int dtype, int64_t tokens, int q_heads, int kv_heads) {
-    const int ns = dense_splits(tokens);
-    return dtype != POPKV_DTYPE_F32 && q_heads == 4 * kv_heads && ns > 0 && ns <= kDenseFusedMaxSplits;
-}
-
-hipError_t launch_attention_dense(const void* queries, int dtype, const void* prefix_k, const void* prefix_v,
-                                  int64_t k_head_stride, int64_t v_head_stride, int64_t tokens, int q_heads,
-                                  int kv_heads, float* partials, hipStream_t stream, const DenseMerge* merge) {
-    const int ns = dense_splits(tokens);
-    switch (dtype) {
-        case POPKV_DTYPE_F32:
-            return launch_dense_t<float>(queries, prefix_k, prefix_v, k_head_stride, v_head_stride, tokens, ns,
-                                         q_heads, kv_heads, partials, merge, stream);
-        case POPKV_DTYPE_F16:
-            return launch_dense_t<f16_t>(queries, prefix_k, prefix_v, k_head_stride, v_head_stride, tokens, ns,
-                                         q_heads, kv_heads, partials, merge, stream);
-        default:
-            return launch_dense_t<bf16_t>(queries, prefix_k, prefix_v, k_head_stride, v_head_stride, tokens, ns,
-                                          q_heads, kv_heads, partials, merge, stream);
-    }
-}
 }  // namespace popkv

@@ -222,32 +222,15 @@ hipError_t launch_layer_step_fused(const void* queries, int dtype, const int32_t
                                    const int64_t* head_to_kv, int q_heads, int kv_heads, float* partials,
                                    int64_t* idx_out, int64_t idx_stride, const void* current_k,
                                    const void* current_v, void* output, hipStream_t stream);
-// Dense attention over every prefix token (head_dim 128, contiguous rows):
-// partials[h][s][130] for dense_splits(tokens) splits of 512 tokens.
-// Query head h reads KV head h / (QH / KVH) (group sizes 1, 2, 4, 8); one
-// workgroup serves a whole group.
-int dense_splits(int64_t tokens);
-// The dense layer's merge fused into its attention launch: tickets[KVH]
-// (zero on entry, left zero), the current token and the output.  Taken when
-// dense_merge_fuses(): fp16 / bf16, GQA groups of 4 (the MFMA kernel), at
-// most 64 splits; otherwise launch_merge_current follows the launch.
-struct DenseMerge {
-    uint32_t* tickets;
-    const void* current_k;
-    const void* current_v;
-    void* output;
-};
-bool dense_merge_fuses(int dtype, int64_t tokens, int q_heads, int kv_heads);
+// Dense attention over every prefix token and the current one (head_dim 128,
+// contiguous rows; tokens may be 0) in one launch: query head h reads KV head
+// h / (QH / KVH) (group sizes 1, 2, 4, 8).  partials: q_heads *
+// dense_max_splits(tokens) states of 130 floats; tickets[KVH]: zero on entry,
+// left zero.
+int64_t dense_max_splits(int64_t tokens);
 hipError_t launch_attention_dense(const void* queries, int dtype, const void* prefix_k, const void* prefix_v,
                                   int64_t k_head_stride, int64_t v_head_stride, int64_t tokens, int q_heads,
-                                  int kv_heads, float* partials, hipStream_t stream,
-                                  const DenseMerge* merge = nullptr);
-
-// Layer-step merge of the split partials plus the current token (head_dim
-// 128); with idx_out non-null, also writes `current` to idx_out[h][idx_slot].
-hipError_t launch_merge_current(const float* partials, int nsplit, const void* queries, int dtype,
-                                const void* current_k, const void* current_v, const int64_t* head_to_kv, int q_heads,
-                                int kv_heads, void* output, int64_t* idx_out, int64_t idx_stride, int64_t idx_slot,
-                                int64_t current, const SeqTable& seq, hipStream_t stream);
+                                  int kv_heads, float* partials, uint32_t* tickets, const void* current_k,
+                                  const void* current_v, void* output, hipStream_t stream);
 
 }  // namespace popkv

@@ -1,0 +1,52 @@
+"""Dense decode attention at the edges of its tiles, waves and splits against
+float64."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from popkv_amd import popkv
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+# Largest error allowed per element: one unit in the last place of the output
+# type (its rounding, and a neighbour where the fp32 result sits on a tie)
+# plus 4e-5: fp32 sums and exponentials of logits up to about 30 in
+# magnitude, relative error about 30 * 2^-23 of values up to about 5.
+ULP = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -23}
+
+
+def _reference(q, pk, pv, k, v):
+    group = q.shape[0] // pk.shape[0]
+    out = []
+    for h in range(q.shape[0]):
+        g = h // group
+        keys = torch.cat([pk[g], k[g, None]]).double()
+        values = torch.cat([pv[g], v[g, None]]).double()
+        out.append(torch.softmax(keys @ q[h].double() / math.sqrt(128), 0) @ values)
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16, torch.float32))
+@pytest.mark.parametrize("group", (1, 2, 4, 8))
+@pytest.mark.parametrize("kv_heads,tokens", [(1, 0), (2, 1), (3, 15), (2, 17), (1, 127), (3, 129), (2, 2049), (40, 1301),
+                                             (1, 40007), (300, 200)])
+def test_dense_attention_tile_and_split_edges(kv_heads, tokens, group, dtype):
+    """No token, a ragged tile, a split of fewer tiles than waves, several
+    splits with a short last one, KV heads that do not divide the workgroup
+    target and more KV heads than it; one workspace used twice (the merge
+    tickets go back to zero)."""
+    gen = torch.Generator().manual_seed(tokens + group)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).to(dtype)  # noqa: E731
+    q, k, v = draw(kv_heads * group, 128) * 3, draw(kv_heads, 128), draw(kv_heads, 128)
+    rows = draw(2, kv_heads, tokens + 3, 128)  # a head stride wider than the prefix
+    pk, pv = rows[0].to(DEV)[:, :tokens], rows[1].to(DEV)[:, :tokens]
+    ws = popkv.LayerStepWorkspace()
+    want = _reference(q, rows[0][:, :tokens], rows[1][:, :tokens], k, v)
+    for _ in range(2):
+        got = popkv.dense_attention_step(q.to(DEV), pk, pv, k.to(DEV), v.to(DEV), workspace=ws)
+        err = (got.cpu().double() - want).abs()
+        assert (err <= ULP[dtype] * want.abs() + 4e-5).all(), float((err - ULP[dtype] * want.abs()).max())
