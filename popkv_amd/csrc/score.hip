@@ -8,16 +8,12 @@
 // popkv_ext.cu:232-281, :911-957) or the production reduction tree (the
 // warp encode inside score(), popkv_ext.cu:677-755).
 //
-// Scorer (head_dim 128): one thread per (KV head, token).  Each thread loads
-// its token's 16-byte sign and magnitude words and its fp16 representatives
-// once with coalesced vector loads, then scores every query head of the GQA
-// group.  The query state of the group is wave-uniform: the kernel reads it
-// with scalar loads, so it lives in SGPRs and the per-head popcount of the
-// query magnitude word is a scalar op.  Per head and representative the
-// kernel needs four signed agreement counts 2*popc(x & sel) - popc(sel)
-// (v_bcnt_u32_b32) and the fp32 fma chain of popkv_ext.cu:502-515 / :867-870,
-// summed from +0 over representatives, times fp32(1/sqrt(128)), rounded once
-// to fp16 (popkv_ext.cu:757-876).
+// Scorer (head_dim 128): the four signed agreement counts 2*popc(x & sel) -
+// popc(sel) of every (query head, token, representative) and the fp32 fma
+// chain of popkv_ext.cu:502-515 / :867-870, summed from +0 over
+// representatives, times fp32(1/sqrt(128)), rounded once to fp16
+// (popkv_ext.cu:757-876).  Two forms, bit for bit alike (score128.h): counts
+// from popcounts, one thread per (KV head, token), or from the matrix cores.
 #include <type_traits>
 
 #include "device_common.h"
@@ -157,6 +153,20 @@ __global__ __launch_bounds__(kScoreThreads) void score_d128_kernel(
                                             ghist, seq, win, blockIdx.x, blockIdx.y);
 }
 
+// The matrix-core form: grid.x token spans, grid.y batch*kv_heads.
+template <int G, int QPK, typename QT>
+__global__ __launch_bounds__(kScoreThreads) void score_d128_mfma_kernel(
+    const int32_t* __restrict__ q_sign, const int32_t* __restrict__ q_mag,
+    const float* __restrict__ q_low, const float* __restrict__ q_delta, const QT* __restrict__ q_raw,
+    const uint4* __restrict__ k_sign, const uint4* __restrict__ k_mag,
+    const uint16_t* __restrict__ k_low, const uint16_t* __restrict__ k_delta,
+    const int64_t* __restrict__ head_to_kv, int q_heads, int kv_heads, int64_t cap, int64_t tokens,
+    uint16_t* __restrict__ scores, int64_t out_stride, uint32_t* __restrict__ ghist, SeqTable seq, int span) {
+    score_mfma_body<G, QPK, QT>(q_sign, q_mag, q_low, q_delta, q_raw, k_sign, k_mag, k_low, k_delta, head_to_kv,
+                                q_heads, kv_heads, cap, tokens, scores, out_stride, ghist, seq, blockIdx.x, span,
+                                blockIdx.y);
+}
+
 // ---------------------------------------------------------------- score, generic D
 
 // One thread per (query row, token), float32 output (popkv_ext.cu:145-230,
@@ -225,6 +235,32 @@ hipError_t launch_encode_g(const T* q, int64_t rows, int d, int g, int order, in
     }
 }
 
+// Tokens of a matrix-core scorer workgroup: whole rounds of 512 (64 per wave), so many
+// that the launch has at most about two workgroups per CU.  Kernel time with
+// 512 / 768 / 1024 / 1536 workgroups wanted (us): 8 sequences x 65535 tokens
+// G64 43.2 / 45.8 / 44.0 / 45.2 and G16 78.2 / 79.7 / 77.8 / 85.0; one of
+// 131071 G64 14.6 / 15.4 / 15.6 / 15.7 and G16 25.4 / 29.5 / 27.4 / 27.9.
+int score_span(int64_t tokens, int64_t rows, bool batched) {
+    constexpr int64_t kRound = kScoreThreads / kWave * kScoreGroup;
+    const int64_t kBlocks = batched ? 1024 : 512;
+    const int64_t per_row = rows < kBlocks ? kBlocks / rows : 1;
+    const int64_t rounds = (tokens + kRound * per_row - 1) / (kRound * per_row);
+    return static_cast<int>(rounds * kRound);
+}
+
+// The matrix-core form: whole lane slots (groups of 4 or 8 heads), where its
+// lower VALU work pays for the LDS exchange and the larger workgroup spans.
+// Scores alone, popcounts / matrix cores (us): 8 heads per group always (G64
+// 4095 tokens x 8 rows 5.25 / 4.90, 65535 12.5 / 9.3; G32 5.96 / 5.27, 14.9 /
+// 12.4; G16 8.2 / 6.7, 24.3 / 20.6), 4 heads at G16 always (5.66 / 5.28, 15.1
+// / 12.7), at G64 and G32 from about 384K (row, token) pairs (262K: layer
+// step 21.2 / 21.6 and 22.2 / 22.0; 524K: 26.2 / 25.7 and 28.5 / 26.9).
+// Groups of 1 or 2 heads would leave lane slots idle or multiply the MFMAs
+// (G16, 1 head, 32767 x 8: 6.2 / 9.9).
+bool score_takes_mfma(int g, int qpk, int64_t row_tokens) {
+    return qpk == 8 || (qpk == 4 && (g == 16 || row_tokens >= 384 * 1024));
+}
+
 template <int G, typename QT>
 hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float* ql, const float* qd, const QT* q_raw,
                                const int32_t* ks, const int32_t* km, const uint16_t* kl, const uint16_t* kd,
@@ -265,6 +301,17 @@ hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float
             case 8: POPKV_SCORE_LAUNCH(8, kWinG); break;
             default: return hipErrorInvalidValue;
         }
+        return hipGetLastError();
+    }
+    if (score_takes_mfma(G, qpk, batch * kvh * tokens)) {
+        const int span = score_span(tokens, batch * kvh, seq.tokens != nullptr);
+        grid.x = static_cast<unsigned>((tokens + span - 1) / span);
+#define POPKV_SCORE_MFMA(Q)                                                                                             \
+    hipLaunchKernelGGL((score_d128_mfma_kernel<G, Q, QT>), grid, dim3(kScoreThreads), 0, stream, qs, qm, ql, qd, q_raw, \
+                       ks4, km4, kl, kd, h2k, qh, kvh, cap, tokens, out, out_stride, ghist, seq, span)
+        if (qpk == 4) POPKV_SCORE_MFMA(4);
+        else POPKV_SCORE_MFMA(8);
+#undef POPKV_SCORE_MFMA
         return hipGetLastError();
     }
     if constexpr (TPT == 2) {

@@ -1,7 +1,8 @@
-// The head_dim-128 popcount scorer's device code: the per-representative
-// count chain, the in-kernel query encode, the tile windows and the scorer
-// body.  score.hip wraps the body in its kernel; the layer step's fused
-// kernel (attention.hip) runs it in its first workgroups.
+// The head_dim-128 scorer's device code: the per-representative count chain,
+// the in-kernel query encode, the tile windows and the popcount scorer's body
+// (score.hip wraps it in its kernel; the layer step's fused kernel,
+// attention.hip, runs it in its first workgroups), and the matrix-core
+// scorer's body.
 #pragma once
 
 #include <type_traits>
@@ -117,10 +118,10 @@ struct __align__(16) HeadState {
     int npq[128 / G];  // -(magnitude bits of representative r)
 };
 
-// Query state of one GQA group in LDS.
-template <int G>
+// Query state of one GQA group of up to HEADS heads in LDS.
+template <int G, int HEADS = kMaxGroupHeads>
 struct GroupState {
-    HeadState<G> h[kMaxGroupHeads];
+    HeadState<G> h[HEADS];
 };
 
 // Encodes the group's query rows (head_dim 128) into `st` in the
@@ -134,8 +135,8 @@ struct GroupState {
 // adding +0 for the other bucket is exact, so this is the reference's fold --
 // and the bucket counts are popcounts of the magnitude words.  All threads of
 // the block call it.
-template <int G, int MAXW>
-__device__ __forceinline__ void encode_group_fold(const float (*qv)[2], int qpk, GroupState<G>& st,
+template <int G, int MAXW, int HEADS>
+__device__ __forceinline__ void encode_group_fold(const float (*qv)[2], int qpk, GroupState<G, HEADS>& st,
                                                   float (*lo_c)[128], float (*hi_c)[128]) {
     constexpr int R = 128 / G;
     const int lane = threadIdx.x & (kWave - 1);
@@ -197,10 +198,10 @@ __device__ __forceinline__ void encode_group_fold(const float (*qv)[2], int qpk,
 }
 
 // Copies a pre-encoded group state from global memory into `st`.
-template <int G>
+template <int G, int HEADS>
 __device__ void load_group_state(const int32_t* __restrict__ q_sign, const int32_t* __restrict__ q_mag,
                                  const float* __restrict__ q_low, const float* __restrict__ q_delta,
-                                 int64_t qrow0, int qpk, GroupState<G>& st) {
+                                 int64_t qrow0, int qpk, GroupState<G, HEADS>& st) {
     constexpr int R = 128 / G;
     for (int i = threadIdx.x; i < qpk * 4; i += kScoreThreads) {
         st.h[i / 4].qs[i % 4] = static_cast<uint32_t>(q_sign[qrow0 * 4 + i]);
@@ -384,6 +385,12 @@ __device__ __forceinline__ void score_d128_body(
 #pragma unroll
     for (int it = 0; it < TPT; ++it) tok[it] = (static_cast<int64_t>(tile) * TPT + it) * kScoreThreads + threadIdx.x;
     load_tokens(slot);
+    // a batched step's tile past its sequence's end: nothing to score, count
+    // or write (the select reads neither its keys nor its window record)
+    if (STEP && seq.tokens != nullptr &&
+        static_cast<int64_t>(tile) * TPT * kScoreThreads >= static_cast<int64_t>(__builtin_amdgcn_readfirstlane(
+            static_cast<int>(min(max(ntok_v, static_cast<int64_t>(0)), tokens)))))
+        return;
 
     __shared__ GroupState<G> st;
     __shared__ uint32_t s_hist[STEP ? (QPK > 0 ? QPK : kMaxGroupHeads) : 1][256];
@@ -550,6 +557,366 @@ __device__ __forceinline__ void score_d128_body(
             if constexpr (WINK) {
                 if (win_on) store_windows();
             }
+        }
+    }
+}
+
+// ---- the matrix-core scorer (GQA groups of 4 or 8 query heads, long rows) ----
+//
+// The four agreement counts of a representative are inner products of small
+// integer vectors over its dimensions: with s = +-1 the sign and m in {0, 1}
+// the magnitude bit of each dimension, and u = s, v = m s,
+//   cs = u_q . u_k, cq = v_q . u_k, ck = u_q . v_k, cqk = v_q . v_k.
+// As FP4 (E2M1: +-1 = 0x2 / 0xa, 0 = 0x0) they are exact operands of
+// v_mfma_f32_16x16x128_f8f6f4 and its fp32 sums (at most 64 in magnitude)
+// are exact, so the scores keep every bit of the popcount form.  One call
+// takes A = 16 query rows (4 lane-group slots x {2 representatives x (u, v)})
+// by B = 16 tokens' u_k, another by their v_k; a representative's row is
+// zero outside its dimensions.  Lane l then holds slot l / 16's eight counts
+// for token l % 16: the fp32 chain follows in registers, no cross-lane step.
+//
+// The lane order of the 128 products does not matter as long as A and B
+// agree: k-group g takes plane word g, and nibble i of operand word j takes
+// bit 4 i + j of it, so expanding a word is a shift and a masked merge per
+// eight dimensions: 18 VALU instructions per 16 tokens and 4 heads, where
+// the counts with v_bcnt took about 45 per (token, head) at G64 (the SIMDs
+// 90 % busy on long batches) and about 190 at G16.
+typedef int mfma_i32x8 __attribute__((ext_vector_type(8)));
+typedef float score_f32x4 __attribute__((ext_vector_type(4)));
+
+struct Fp4Words {
+    uint32_t w[4];
+};
+// u = +-1 per dimension of a sign word (a set bit as 0xa on both sides: the
+// products only see whether the signs agree)
+__device__ __forceinline__ Fp4Words fp4_signs(uint32_t sign) {
+    Fp4Words r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r.w[j] = ((sign << (3 - j)) & 0x88888888u) | 0x22222222u;
+    return r;
+}
+// v = u where the magnitude bit is set, else +-0
+__device__ __forceinline__ Fp4Words fp4_magnitudes(uint32_t sign, uint32_t mag) {
+    Fp4Words r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        r.w[j] = ((sign << (3 - j)) & 0x88888888u) | ((j < 2 ? mag << (1 - j) : mag >> (j - 1)) & 0x22222222u);
+    return r;
+}
+__device__ __forceinline__ score_f32x4 mfma_fp4(const Fp4Words& a, const Fp4Words& b, score_f32x4 c) {
+    mfma_i32x8 x = {}, y = {};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        x[j] = static_cast<int>(a.w[j]);
+        y[j] = static_cast<int>(b.w[j]);
+    }
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, y, c, 4, 4, 0, 0, 0, 0);  // FP4 by FP4, unscaled
+}
+
+// The A operand of representatives 2 set and 2 set + 1 for this lane: row
+// l % 16 = 4 slot + 2 (rep of the pair) + (0: u, 1: v), plane word l / 16,
+// slot's query head h0 + slot.
+template <int G, int HEADS>
+__device__ __forceinline__ Fp4Words query_rows(const GroupState<G, HEADS>& st, int set, int h0) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int g = lane >> 4, row = lane & 15, rep = (row >> 1) & 1;
+    const HeadState<G>& h = st.h[h0 + (row >> 2)];
+    const uint32_t qs = h.qs[g], qm = h.qm[g];
+    Fp4Words r = (row & 1) ? fp4_magnitudes(qs, qm) : fp4_signs(qs);
+    const bool in = G == 64 ? g / 2 == rep : G == 32 ? g == 2 * set + rep : g == set;
+    // (G16: the pair shares a word, its low and its high 16 dimensions)
+    const uint32_t keep = !in ? 0u : G == 16 ? (rep ? 0xffff0000u : 0x0000ffffu) : 0xffffffffu;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r.w[j] &= keep;
+    return r;
+}
+
+// Lane-row moves (rows of 16 lanes): a's odd rows exchanged with b's even
+// ones, a's upper half with b's lower half.
+__device__ __forceinline__ void row_swap16(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void row_swap32(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+// x[w] of lane row r becomes x[r] of lane row w (word w of token 16 r + c to
+// word r of set w).
+__device__ __forceinline__ void rows_transpose(uint32_t (&x)[4]) {
+    row_swap32(x[0], x[2]);
+    row_swap32(x[1], x[3]);
+    row_swap16(x[0], x[1]);
+    row_swap16(x[2], x[3]);
+}
+
+constexpr int kScoreGroup = 64;  // tokens a wave loads and scores at a time
+
+// Orders this wave's LDS accesses before and after: one wave's LDS
+// operations complete in order, so only the compiler is held.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The scorer's workgroup: tokens [t_begin, t_begin + span) of block row
+// `grow` (sequence, KV group slot; batch * kv_heads rows), span a multiple
+// of 512.  QT is the raw query
+// type when the kernel encodes the query itself (layer step), void when it
+// reads a pre-encoded state.  Wave w takes the span's groups of 64 tokens w,
+// w + 8, ..., each loaded with one 16-byte word per lane and plane a group
+// ahead of its use, spread to the operand layout by lane-row swaps, and
+// leaving through the wave's own strip of LDS in whole 16-byte words: no
+// barrier between the encode and the histogram's end.
+//
+// The scorer streams KVH (32 + 4 R) bytes per token, so on long rows a
+// workgroup per tile would have every workgroup load at once, then all
+// compute, and pay the query's load and encode (about 2 us) per tile; here
+// the launch gives each CU two workgroups whose spans cover the rows.  Kernel
+// time before (popcounts, a workgroup per tile) -> now, 32 query heads over 8
+// KV heads: 131071 tokens G64 16.9 -> 14.6 us (3.4 TB/s of 50 MB), G16 35.4
+// -> 25.4; 8 x 65535 tokens G64 47.8 -> 43.2 us (4.6 TB/s of 201 MB).
+template <int G, int QPK, typename QT>
+__device__ __forceinline__ void score_mfma_body(
+    const int32_t* __restrict__ q_sign, const int32_t* __restrict__ q_mag,
+    const float* __restrict__ q_low, const float* __restrict__ q_delta, const QT* __restrict__ q_raw,
+    const uint4* __restrict__ k_sign, const uint4* __restrict__ k_mag,
+    const uint16_t* __restrict__ k_low, const uint16_t* __restrict__ k_delta,
+    const int64_t* __restrict__ head_to_kv, int q_heads, int kv_heads,
+    int64_t cap, int64_t tokens, uint16_t* __restrict__ scores, int64_t out_stride,
+    uint32_t* __restrict__ ghist, SeqTable seq, uint32_t tile, int span, uint32_t grow_u) {
+    static_assert(QPK == 4 || QPK == 8, "a query head per lane slot of a C matrix");
+    constexpr bool STEP = !std::is_void_v<QT>;
+    constexpr int R = 128 / G, NS = R / 2;  // representatives, and pairs of them
+    constexpr int HS = QPK / 4;             // C matrices per 16 tokens
+    constexpr int WAVES = kScoreThreads / kWave;
+    args_in_sgprs(head_to_kv, k_sign, k_mag, k_low, k_delta, q_heads, kv_heads, cap, tokens, seq.tokens,
+                  seq.cache_rows);
+    if constexpr (STEP) args_in_sgprs(q_raw);
+    // block row (sequence b, KV group slot): 32-bit arithmetic, the row
+    // count being below 2^31
+    const int grow = static_cast<int>(grow_u);
+    const int bi = div_nonneg(grow, kv_heads);
+    const int kv_slot = grow - bi * kv_heads;
+    const int64_t b = bi;
+    const int64_t qh0 = static_cast<int64_t>(kv_slot) * QPK;
+    const int64_t qrow0 = b * q_heads + qh0;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+
+    // Loads, in issue order (they retire in that order, vmcnt): the raw
+    // query values the encode needs; the group's KV mapping and (batched)
+    // the sequence's token count, as vector loads at a lane-opaque zero
+    // offset (as scalar loads their wait would also hold back the query
+    // loads); then this lane's token of the wave's first group at the KV head
+    // the mapping names for the standard grouping, head_to_kv[qh0] = kv_slot,
+    // so that their latency overlaps the encode.  Once the mapping has
+    // arrived, a group that maps elsewhere (clamped into [0, kv_heads), never
+    // dereferenced outside) loads its rows again.
+    constexpr int MAXW = (QPK + WAVES - 1) / WAVES;
+    float qv[MAXW][2];
+    if constexpr (STEP) {
+#pragma unroll
+        for (int i = 0; i < MAXW; ++i) {
+            const int h = min(wave + i * WAVES, QPK - 1);
+            const QT* src = q_raw + (qrow0 + h) * 128;
+            qv[i][0] = Elem<QT>::load(src, lane);
+            qv[i][1] = Elem<QT>::load(src, lane + 64);
+        }
+    }
+    int z = 0;
+    asm volatile("" : "+v"(z));
+    const int64_t map_v = head_to_kv[qh0 + z];
+    const int64_t ntok_v = seq.tokens != nullptr ? seq.tokens[b + z] : tokens;
+    const int64_t t_begin = static_cast<int64_t>(tile) * span;
+    struct Group {
+        uint32_t s[4], m[4], l[NS], d[NS];
+    };
+    // this lane's token of the group at t_begin + 64 i (a batched step gives
+    // each sequence its own cache; the reference's batch shares one); the
+    // loads stay within the launch bound `tokens`
+    int64_t cbase = b * seq.cache_rows + kv_slot * cap;
+    auto load_group = [&](int i, Group& k) {
+        const int64_t krow = cbase + min(t_begin + i * kScoreGroup + lane, tokens - 1);
+        const uint4 s4 = k_sign[krow], m4 = k_mag[krow];
+        k.s[0] = s4.x; k.s[1] = s4.y; k.s[2] = s4.z; k.s[3] = s4.w;
+        k.m[0] = m4.x; k.m[1] = m4.y; k.m[2] = m4.z; k.m[3] = m4.w;
+        if constexpr (NS == 1) {
+            k.l[0] = reinterpret_cast<const uint32_t*>(k_low)[krow];
+            k.d[0] = reinterpret_cast<const uint32_t*>(k_delta)[krow];
+        } else if constexpr (NS == 2) {
+            const uint2 l2 = reinterpret_cast<const uint2*>(k_low)[krow], d2 = reinterpret_cast<const uint2*>(k_delta)[krow];
+            k.l[0] = l2.x; k.l[1] = l2.y;
+            k.d[0] = d2.x; k.d[1] = d2.y;
+        } else {
+            const uint4 l4 = reinterpret_cast<const uint4*>(k_low)[krow], d4 = reinterpret_cast<const uint4*>(k_delta)[krow];
+            k.l[0] = l4.x; k.l[1] = l4.y; k.l[2] = l4.z; k.l[3] = l4.w;
+            k.d[0] = d4.x; k.d[1] = d4.y; k.d[2] = d4.z; k.d[3] = d4.w;
+        }
+    };
+    Group cur;
+    load_group(wave, cur);
+    const int64_t ntok_b = min(max(ntok_v, static_cast<int64_t>(0)), tokens);
+    // a batched step's span past its sequence's end: nothing to score, count
+    // or write (the select reads neither its keys nor its window record)
+    if (STEP && seq.tokens != nullptr &&
+        t_begin >= static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(ntok_b))))
+        return;
+
+    __shared__ GroupState<G, QPK> st;
+    __shared__ uint32_t s_hist[STEP ? QPK : 1][256];
+    // each wave's outputs of its current group; rows 32 bytes apart modulo
+    // the LDS banks (the four slots of a wave write four heads at once)
+    constexpr int KROW = WAVES * kScoreGroup + 16;
+    __shared__ __align__(16) uint16_t s_keys[QPK][KROW];
+    __shared__ __align__(16) uint32_t s_rep[WAVES][kScoreGroup * 2 * NS];
+    if constexpr (STEP) {
+        for (int i = threadIdx.x; i < QPK * 256; i += kScoreThreads) (&s_hist[0][0])[i] = 0u;
+    }
+    if constexpr (!STEP) {
+        load_group_state<G>(q_sign, q_mag, q_low, q_delta, qrow0, QPK, st);
+    } else {
+        __shared__ __align__(16) float lo_c[QPK][128];
+        __shared__ __align__(16) float hi_c[QPK][128];
+        encode_group_fold<G, MAXW>(qv, QPK, st, lo_c, hi_c);
+    }
+    {
+        const int m = __builtin_amdgcn_readfirstlane(static_cast<int>(min(max(map_v, static_cast<int64_t>(0)),
+                                                                          static_cast<int64_t>(kv_heads - 1))));
+        if (m != kv_slot) {
+            cbase = b * seq.cache_rows + m * cap;
+            load_group(wave, cur);
+        }
+    }
+    const int slot = lane >> 4, tcol = lane & 15;
+    Fp4Words qa[HS][NS];
+    float ql[HS][R], dq[HS][R];
+#pragma unroll
+    for (int hs = 0; hs < HS; ++hs) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) qa[hs][s] = query_rows<G, QPK>(st, s, hs * 4);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            ql[hs][r] = st.h[hs * 4 + slot].ql[r];
+            dq[hs][r] = st.h[hs * 4 + slot].qd[r];
+        }
+    }
+    // (the span's tokens and groups, block-uniform)
+    const int nloc = __builtin_amdgcn_readfirstlane(static_cast<int>(min(ntok_b - t_begin, static_cast<int64_t>(span))));
+    const int ngroups = (nloc + kScoreGroup - 1) / kScoreGroup;
+    for (int g = wave; g < ngroups; g += WAVES) {
+        Group next;
+        if (g + WAVES < ngroups) load_group(g + WAVES, next);
+        // the planes' words to the operand layout: set i's word l / 16 of token l % 16
+        rows_transpose(cur.s);
+        rows_transpose(cur.m);
+        // low / delta through the wave's strip: every lane slot reads its token's
+        {
+            uint32_t* rep = &s_rep[wave][lane * 2 * NS];
+            if constexpr (NS == 1) {
+                *reinterpret_cast<uint2*>(rep) = make_uint2(cur.l[0], cur.d[0]);
+            } else if constexpr (NS == 2) {
+                *reinterpret_cast<uint4*>(rep) = make_uint4(cur.l[0], cur.l[1], cur.d[0], cur.d[1]);
+            } else {
+                reinterpret_cast<uint4*>(rep)[0] = make_uint4(cur.l[0], cur.l[1], cur.l[2], cur.l[3]);
+                reinterpret_cast<uint4*>(rep)[1] = make_uint4(cur.d[0], cur.d[1], cur.d[2], cur.d[3]);
+            }
+        }
+        wave_lds_order();
+        const bool whole = nloc - g * kScoreGroup >= kScoreGroup;  // uniform
+        const int col0 = wave * kScoreGroup;  // of the group in s_keys
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int tg = 16 * u + tcol;  // this lane's token in the group
+            float kl[R], dk[R];
+            {
+                const uint32_t* rep = &s_rep[wave][tg * 2 * NS];
+                uint32_t w[2 * NS];
+                if constexpr (NS == 1) {
+                    const uint2 x = *reinterpret_cast<const uint2*>(rep);
+                    w[0] = x.x; w[1] = x.y;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NS / 2; ++i) {
+                        const uint4 x = reinterpret_cast<const uint4*>(rep)[i];
+                        w[4 * i] = x.x; w[4 * i + 1] = x.y; w[4 * i + 2] = x.z; w[4 * i + 3] = x.w;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < NS; ++i) {
+                    kl[2 * i] = bits_f16(w[i] & 0xffffu); kl[2 * i + 1] = bits_f16(w[i] >> 16);
+                    dk[2 * i] = bits_f16(w[NS + i] & 0xffffu); dk[2 * i + 1] = bits_f16(w[NS + i] >> 16);
+                }
+            }
+            const Fp4Words ku = fp4_signs(cur.s[u]), kv = fp4_magnitudes(cur.s[u], cur.m[u]);
+#pragma unroll
+            for (int hs = 0; hs < HS; ++hs) {
+                float total = 0.0f;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const score_f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                    const score_f32x4 cu = mfma_fp4(qa[hs][s], ku, zero), cv = mfma_fp4(qa[hs][s], kv, zero);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int r = 2 * s + i;
+                        total = total + fmaf(ql[hs][r] * kl[r], cu[2 * i],
+                                             fmaf(dq[hs][r] * kl[r], cu[2 * i + 1],
+                                                  fmaf(ql[hs][r] * dk[r], cv[2 * i], dq[hs][r] * dk[r] * cv[2 * i + 1])));
+                    }
+                }
+                const float sc = total * 0x1.6a09e6p-4f;  // fp32(1/sqrt(128)) = 0x3DB504F3
+                const uint32_t bits = f16_rne(sc);
+                uint32_t key = bits;
+                if constexpr (STEP) {
+                    // order_key(bits): b ^ (s | 0x8000) with s = bit 15
+                    // sign-extended -- every bit flips for a negative value, only
+                    // bit 15 for a non-negative one; the bits above 15 are left
+                    // as garbage (the store keeps 16 bits, the histogram takes
+                    // bits 8..15).  The NaN test is done on the fp32 value (an
+                    // fp32 NaN is exactly an fp16 NaN after the conversion).
+                    const uint32_t sgn = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int32_t>(bits), 15, 1));
+                    key = sc != sc ? 0xffffu : bits ^ (sgn | 0x8000u);
+                    // (tokens past the end score the clamped last row: key 0, not counted)
+                    if (whole || g * kScoreGroup + tg < nloc) atomicAdd(&s_hist[hs * 4 + slot][(key >> 8) & 0xffu], 1u);
+                    else key = 0u;
+                }
+                s_keys[hs * 4 + slot][col0 + tg] = static_cast<uint16_t>(key);
+            }
+        }
+        wave_lds_order();
+        const int64_t t0 = t_begin + g * kScoreGroup;
+        const int left = nloc - g * kScoreGroup;
+        if constexpr (!STEP) {
+            // fp16 scores at any row stride and alignment: two bytes a lane,
+            // 128 contiguous bytes a wave store
+#pragma unroll
+            for (int h = 0; h < QPK; ++h)
+                if (lane < left) scores[(qrow0 + h) * out_stride + t0 + lane] = s_keys[h][col0 + lane];
+        } else {
+            // key rows: padded to a multiple of 128 keys and 16-byte aligned,
+            // so the last, partly filled 8 bytes stay inside the row.  Written
+            // through to memory (device-coherent stores), 128 contiguous bytes
+            // a head.
+#pragma unroll
+            for (int h0 = 0; h0 < QPK; h0 += 4) {  // 16 lanes a head, 8 bytes a lane
+                const int h = h0 + (lane >> 4), t = 4 * (lane & 15);
+                if (h < QPK && t < left)
+                    __hip_atomic_store(reinterpret_cast<uint64_t*>(scores + (qrow0 + h) * out_stride + t0 + t),
+                                       *reinterpret_cast<const uint64_t*>(&s_keys[h][col0 + t]), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        wave_lds_order();
+        cur = next;
+    }
+    if constexpr (STEP) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < QPK * 256; i += kScoreThreads) {
+            const uint32_t c = (&s_hist[0][0])[i];
+            if (c != 0u) atomicAdd(&ghist[(qrow0 + i / 256) * 256 + (i & 255)], c);
         }
     }
 }
