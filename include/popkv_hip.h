@@ -282,6 +282,21 @@ int popkv_decode_layer_batched(const void* queries, int32_t dtype,
                                int64_t* indices_out, int64_t index_row_stride, int32_t* status,
                                void* workspace, size_t workspace_bytes, void* stream);
 
+/* The per-token metadata append of several layers at one point of their
+ * token groups (append_retrieval_caches, popkv.py:883-942: torch.cat staging
+ * and pack_keys_into for every layer), one launch per 32 layers.  Host arrays
+ * of `layers` device pointers: active[l] [KVH, active_tokens, 128] (may be
+ * NULL when active_tokens is 0), new_k[l] [KVH, 128], staged[l]
+ * [KVH, active_tokens + 1, 128] (written: the active keys and the new one)
+ * and the layer's packed planes [KVH, capacity, .], whose rows
+ * [sealed_tokens, sealed_tokens + active_tokens] are re-encoded.
+ * active_tokens < token_group_size; all 16-byte aligned; no two layers may
+ * share planes or staged rows. */
+int popkv_stage_append(const void* const* active, const void* const* new_k, void* const* staged,
+                       int32_t* const* k_sign, int32_t* const* k_mag, void* const* k_low, void* const* k_delta,
+                       int64_t layers, int32_t dtype, int64_t kv_heads, int64_t active_tokens, int64_t capacity,
+                       int64_t sealed_tokens, int32_t token_group_size, int32_t dim_group_size, void* stream);
+
 /* Allocation-free form of popkv_layer_step: the same kernels and results,
  * with the workspace taken from a library-owned device array of
  * POPKV_LAYER_STEP_SCRATCH_BYTES per GPU (a file-scope __device__ array,

@@ -62,6 +62,8 @@ _SIGNATURES = {
                                                   _vp, _vp, _c_i64, _vp, _vp, _c_size, _vp]),
     "popkv_append": (ctypes.c_int, [_vp, _vp, _c_i32, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_i64,
                                     _c_i64, _c_i32, _c_i32, _vp, _vp]),
+    "popkv_stage_append": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i32, _c_i64, _c_i64, _c_i64,
+                                          _c_i64, _c_i32, _c_i32, _vp]),
     "popkv_layer_step_scratch_bytes": (_c_size, []),
     "popkv_layer_step_noalloc": (ctypes.c_int, [_vp, _c_i32, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64,
                                                 _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _vp, _vp, _vp]),
@@ -108,6 +110,11 @@ def dtype_code(t: torch.Tensor) -> int:
 
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
+
+
+def pointer_array(pointers: list[int]) -> ctypes.Array:
+    """A host array of device pointers."""
+    return (_vp * len(pointers))(*pointers)
 
 
 def stream_of(device: torch.device) -> int:

@@ -706,6 +706,51 @@ int popkv_append(const void* new_k, const void* new_v, int32_t dtype, void* key_
                     "popkv_append");
 }
 
+int popkv_stage_append(const void* const* active, const void* const* new_k, void* const* staged,
+                       int32_t* const* k_sign, int32_t* const* k_mag, void* const* k_low, void* const* k_delta,
+                       int64_t layers, int32_t dtype, int64_t kv_heads, int64_t active_tokens, int64_t capacity,
+                       int64_t sealed_tokens, int32_t token_group_size, int32_t dim_group_size, void* stream) {
+    if (!active || !new_k || !staged || !k_sign || !k_mag || !k_low || !k_delta)
+        return fail(POPKV_ERR_INVALID, "null pointer");
+    if (!valid_dtype(dtype)) return fail(POPKV_ERR_INVALID, "keys must be fp32/fp16/bf16");
+    if (layers < 0 || kv_heads <= 0 || kv_heads > 65535) return fail(POPKV_ERR_INVALID, "bad layer or KV head count");
+    if (token_group_size < 1 || token_group_size > 4096)
+        return fail(POPKV_ERR_INVALID, "token_group_size must be between 1 and 4096");
+    if (!valid_group(dim_group_size)) return fail(POPKV_ERR_INVALID, "dim_group_size must be 16, 32, or 64");
+    if (active_tokens < 0 || active_tokens >= token_group_size)
+        return fail(POPKV_ERR_INVALID, "the active group has no room for another token");
+    if (sealed_tokens < 0 || sealed_tokens + active_tokens + 1 > capacity)
+        return fail(POPKV_ERR_CAPACITY, "Pop-KV cache capacity exceeded");
+    for (int64_t i = 0; i < layers; ++i) {
+        const void* p[] = {new_k[i], staged[i], k_sign[i], k_mag[i], k_low[i], k_delta[i]};
+        for (const void* q : p) {
+            if (!q) return fail(POPKV_ERR_INVALID, "null pointer");
+            if (!aligned16(q)) return fail(POPKV_ERR_UNSUPPORTED, "append tensors need 16-byte alignment");
+        }
+        if (active_tokens > 0 && (!active[i] || !aligned16(active[i])))
+            return fail(POPKV_ERR_UNSUPPORTED, "append tensors need 16-byte alignment");
+    }
+    for (int64_t l0 = 0; l0 < layers; l0 += popkv::kStageLayers) {
+        const int n = static_cast<int>(layers - l0 < popkv::kStageLayers ? layers - l0 : popkv::kStageLayers);
+        popkv::StagePointers t{};
+        for (int i = 0; i < n; ++i) {
+            t.active[i] = active[l0 + i];
+            t.new_k[i] = new_k[l0 + i];
+            t.staged[i] = staged[l0 + i];
+            t.k_sign[i] = k_sign[l0 + i];
+            t.k_mag[i] = k_mag[l0 + i];
+            t.k_low[i] = k_low[l0 + i];
+            t.k_delta[i] = k_delta[l0 + i];
+        }
+        const int st = launched(popkv::launch_stage_append(t, n, dtype, static_cast<int>(kv_heads),
+                                                           static_cast<int>(active_tokens), capacity, sealed_tokens,
+                                                           token_group_size, dim_group_size, as_stream(stream)),
+                                "popkv_stage_append");
+        if (st) return st;
+    }
+    return POPKV_OK;
+}
+
 int popkv_layer_step_attention(const void* queries, int32_t dtype, const void* prefix_k, const void* prefix_v,
                                int64_t k_head_stride, int64_t v_head_stride, const int64_t* head_to_kv,
                                int64_t q_heads, int64_t kv_heads, int64_t tokens, int64_t budget,

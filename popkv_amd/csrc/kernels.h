@@ -49,6 +49,24 @@ hipError_t launch_append(const void* new_k, const void* new_v, int dtype, void* 
                          int32_t* k_mag, uint16_t* k_low, uint16_t* k_delta, int64_t capacity,
                          int token_group_size, int dim_group_size, int32_t* status, hipStream_t stream);
 
+// Per-token append of several layers whose active groups hold the same number
+// of keys (head_dim 128), one launch per kStageLayers layers: for every layer
+// and KV head, staged = active (n rows) and the new key, and the n + 1 rows
+// (one token group at most) encoded into packed rows sealed .. sealed + n.
+constexpr int kStageLayers = 32;
+struct StagePointers {
+    const void* active[kStageLayers];  // [KVH, n, 128]
+    const void* new_k[kStageLayers];   // [KVH, 128]
+    void* staged[kStageLayers];        // [KVH, n + 1, 128]
+    int32_t* k_sign[kStageLayers];
+    int32_t* k_mag[kStageLayers];
+    void* k_low[kStageLayers];
+    void* k_delta[kStageLayers];
+};
+hipError_t launch_stage_append(const StagePointers& ptrs, int layers, int dtype, int kv_heads, int active_tokens,
+                               int64_t capacity, int64_t sealed, int token_group_size, int dim_group_size,
+                               hipStream_t stream);
+
 hipError_t launch_query_encode(const void* queries, int dtype, int64_t rows, int head_dim,
                                int dim_group_size, int order, int32_t* q_sign, int32_t* q_mag,
                                float* q_low, float* q_delta, hipStream_t stream);

@@ -3,7 +3,8 @@
 The PopKV part of the reference's ``popkv.py``, with the same names and
 semantics: presets and ``RetrievalConfig`` (popkv.py:18-64), ``PopKVCache``
 with prefix prepack and per-token append (popkv.py:89-96, :414-459), the
-batched append phases of ``append_retrieval_caches`` (popkv.py:883-942), the
+batched append phases of ``append_retrieval_caches`` (popkv.py:883-942; one
+native call for caches at the same point of their token groups), the
 static K/V cache append (popkv.py:105-111, :964-972), ``_append_current`` /
 ``_sparse_layer_indices`` (popkv.py:283-291), and the PopKV branch of
 ``LlamaSparseDecoder.decode`` (popkv.py:1076-1115) as ``popkv_retrieval_step``.
@@ -179,6 +180,53 @@ def build_retrieval_caches(layer_keys: dict[int, torch.Tensor], *, method: str,
         for layer, keys in layer_keys.items()})
 
 
+def _stage_append(items: list[tuple[PopKVCache, torch.Tensor]]) -> bool:
+    """The three phases of append_retrieval_caches in one native call, for
+    caches that stand at the same point of equal token groups: head_dim 128,
+    distinct contiguous planes on one GPU, contiguous 16-byte aligned keys of
+    one dtype, room for the token.  Returns False, with nothing done, for
+    anything else (the general path then appends or raises)."""
+    if not items:
+        return False
+    first, key = items[0]
+    n, tg, g = int(first.active_keys.shape[1]), first.group_size, first.dim_group_size
+    if key.ndim != 3 or key.shape[2] != 128 or not key.is_cuda or key.dtype not in nat._DTYPES:
+        return False
+    kv_heads, dev, dtype = int(key.shape[0]), key.device, key.dtype
+    capacity = int(first.packed[0].shape[1])
+    sealed = first.sealed_tokens
+    if g not in (16, 32, 64) or not 1 <= tg <= MAX_TOKEN_GROUP_SIZE or (g != 32 and tg not in SPECIALIZED_TOKEN_GROUP_SIZES) \
+            or n >= tg or sealed < 0 or sealed + n + 1 > capacity or kv_heads < 1:
+        return False
+    shapes = ((kv_heads, n, 128), (kv_heads, 1, 128)) + ((kv_heads, capacity, 4),) * 2 + ((kv_heads, capacity, 128 // g),) * 2
+    dtypes = (dtype, dtype, torch.int32, torch.int32, torch.float16, torch.float16)
+    columns: tuple[list[int], ...] = ([], [], [], [], [], [])
+    for cache, key in items:
+        if cache.sealed_tokens != sealed or cache.group_size != tg or cache.dim_group_size != g or len(cache.packed) != 4:
+            return False
+        for t, shape, dt, column in zip((cache.active_keys, key, *cache.packed), shapes, dtypes, columns):
+            if t.shape != shape or t.dtype != dt or t.device != dev or not t.is_contiguous():
+                return False
+            p = t.data_ptr()
+            if p % 16:
+                return False
+            column.append(p)
+    if any(len(set(column)) != len(items) for column in columns[2:]) or len({id(cache) for cache, _ in items}) != len(items):
+        return False
+    with torch.cuda.device(dev):
+        staged = torch.empty((len(items), kv_heads, n + 1, 128), device=dev, dtype=dtype).unbind(0)
+        active, new_k, *planes = columns
+        nat.call("popkv_stage_append", *map(nat.pointer_array, (active, new_k, [t.data_ptr() for t in staged], *planes)),
+                 len(items), nat._DTYPES[dtype], kv_heads, n, capacity, sealed, tg, g, nat.stream_of(dev))
+    for (cache, _), keys in zip(items, staged):
+        cache.active_keys = keys
+        cache.token_count += 1
+        if n + 1 == tg:
+            cache.sealed_tokens += tg
+            cache.active_keys = keys[:, :0].contiguous()
+    return True
+
+
 def append_retrieval_caches(caches: RetrievalCaches, new_keys: Sequence[torch.Tensor], *,
                             timer=None) -> None:
     """Batched per-token append across layers in three phases -- stage all,
@@ -188,6 +236,8 @@ def append_retrieval_caches(caches: RetrievalCaches, new_keys: Sequence[torch.Te
     for layer, cache in caches.layers.items():
         k = new_keys[layer]
         items.append((cache, k[0] if k.ndim == 4 else k))
+    if timer is None and _stage_append(items):
+        return
     for cache, keys in items:
         cache.active_keys = torch.cat([cache.active_keys, keys.detach()], dim=1).contiguous()
         if cache.sealed_tokens + int(cache.active_keys.shape[1]) > int(cache.packed[0].shape[1]):
