@@ -8,9 +8,11 @@
 // its token group come first (thresholds 0.5*max / 0.5*min in LDS), then one
 // token per lane: the sign/magnitude words and the representatives, reduced
 // in one lane's registers in the production tree order, so the bit-exact
-// sums need no cross-lane shuffles.  Other head sizes (pack_kernel) use 256
-// threads per group: per-dimension extrema by (dimension, token stripe),
-// then one token per thread.
+// sums need no cross-lane shuffles.  Other head sizes of whole 32-dimension
+// words: pack_rows_kernel, one workgroup per 64 rows, a lane per (token,
+// chunk).  Everything else (pack_kernel) uses 256 threads per group:
+// per-dimension extrema by (dimension, token stripe), then one token per
+// thread.
 //
 // Semantics follow the reference packers: popkv_ext.cu:79-143 (G32),
 // :376-500 (fused G16/G64, head_dim 128), :283-374 (generic G16/G64), with
@@ -26,6 +28,7 @@ namespace popkv {
 namespace {
 
 constexpr int kPackThreads = 256;
+constexpr int kMaxStaticLds = 64 * 1024;  // LDS a launch may ask for without an attribute
 
 // Encodes one chunk of CH = max(G, 32) dimensions of one token.
 // dims [c0, c0 + CH); `valid_d` = number of real dims in the head.
@@ -182,6 +185,128 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
     }
 }
 
+// Two consecutive elements at an address aligned to the pair.
+__device__ __forceinline__ float2 load_pair(const float* p) { return *reinterpret_cast<const float2*>(p); }
+__device__ __forceinline__ float2 load_pair(const bf16_t* p) {
+    const uint32_t u = *reinterpret_cast<const uint32_t*>(p);
+    return make_float2(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u));
+}
+__device__ __forceinline__ float2 load_pair(const f16_t* p) {
+    const uint32_t u = *reinterpret_cast<const uint32_t*>(p);
+    return make_float2(bits_f16(u & 0xffffu), bits_f16(u >> 16));
+}
+
+constexpr int kRowsBlock = 64;  // rows a workgroup of pack_rows_kernel takes at most
+constexpr int kRowsStripe = 8;  // rows per extrema stripe
+
+// LDS of pack_rows_kernel: the rows (16 bytes of padding each, so that lanes
+// at one offset of neighbouring rows spread over the banks), the stripes'
+// maxima and minima (4 floats of padding), and the packed rows.
+__host__ __device__ constexpr int pack_rows_pitch(int d, int esize) { return d * esize + 16; }
+__host__ __device__ constexpr int pack_rows_ext(int d) { return kRowsBlock / kRowsStripe * (d + 4); }
+__host__ __device__ constexpr int pack_rows_lds(int d, int g, int esize) {
+    return kRowsBlock * pack_rows_pitch(d, esize) + 2 * pack_rows_ext(d) * 4 + kRowsBlock * (2 * (d / 32) * 4 + 2 * (d / g) * 2);
+}
+
+// Prepack of head sizes other than 128 that whole chunks of CH = max(G, 32)
+// dimensions fill: block (x, y) encodes rows [rpb x, rpb x + rpb) of KV head y,
+// rpb the whole token groups (a multiple of 8 tokens each) within 64 rows.  A
+// workgroup per token group that read each row by single elements, once for
+// the extrema and once a lane, was bound by the latency of those loads with
+// 32-token groups filling 32 of 256 encode lanes.  Here the rows cross memory
+// once, 16 bytes a lane, into LDS; extrema run over stripes of 8 rows there;
+// each (row, chunk) is a lane's; and the packed rows leave whole.
+// Measured (8 heads, graph replay, the general kernel -> this one): 64
+// dimensions, G32 / 32 tokens fp16, 8191 tokens 25.0 -> 8.3 us, 1000 tokens
+// 20.2 -> 7.3; 96 dimensions, 16383 tokens, G16 / 32 tokens fp16 76.4 -> 19.5,
+// G32 / 64 tokens bf16 63.6 -> 22.3; 64 dimensions, G64 / 64 tokens fp32, 16384
+// tokens 53.0 -> 32.3; 256 dimensions, G32 / 32 tokens bf16, 8191 tokens 104 ->
+// 29.7.
+template <typename T, int G>
+__global__ __launch_bounds__(kPackThreads) void pack_rows_kernel(
+    const T* __restrict__ keys, int64_t head_stride, int64_t tokens, int d, int tg, int rpb,
+    int32_t* __restrict__ k_sign, int32_t* __restrict__ k_mag, uint16_t* __restrict__ k_low,
+    uint16_t* __restrict__ k_delta, int64_t cap, int64_t offset) {
+    constexpr int CH = G > 32 ? G : 32;
+    extern __shared__ __align__(16) char lds[];
+    const int w = d / 32, r = d / G, pitch = pack_rows_pitch(d, sizeof(T)), ext_pitch = d + 4;
+    float* s_mx = reinterpret_cast<float*>(lds + kRowsBlock * pitch);
+    float* s_mn = s_mx + pack_rows_ext(d);
+    uint32_t* s_sign = reinterpret_cast<uint32_t*>(s_mn + pack_rows_ext(d));
+    uint32_t* s_mag = s_sign + kRowsBlock * w;
+    uint16_t* s_low = reinterpret_cast<uint16_t*>(s_mag + kRowsBlock * w);
+    uint16_t* s_delta = s_low + kRowsBlock * r;
+
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int64_t kvh = blockIdx.y, gs = static_cast<int64_t>(blockIdx.x) * rpb;
+    const int n = static_cast<int>(min(static_cast<int64_t>(rpb), tokens - gs));
+    const uint4* src = reinterpret_cast<const uint4*>(keys + kvh * head_stride + gs * d);
+    const int vpr = d * static_cast<int>(sizeof(T)) / 16;
+    for (int i = tid; i < n * vpr; i += nt)
+        *reinterpret_cast<uint4*>(lds + i / vpr * pitch + i % vpr * 16) = src[i];
+    __syncthreads();
+
+    // extrema of each stripe and pair of dimensions
+    const int stripes = (n + kRowsStripe - 1) / kRowsStripe, pairs = d / 2;
+    for (int i = tid; i < stripes * pairs; i += nt) {
+        const int st = i / pairs, dim = i % pairs * 2, t0 = st * kRowsStripe;
+        float2 mx = make_float2(-INFINITY, -INFINITY), mn = make_float2(INFINITY, INFINITY);
+#pragma unroll
+        for (int j = 0; j < kRowsStripe; ++j) {
+            // past the end: the last row again
+            const float2 x = load_pair(reinterpret_cast<const T*>(lds + min(t0 + j, n - 1) * pitch) + dim);
+            mx = make_float2(fmaxf(mx.x, x.x), fmaxf(mx.y, x.y));
+            mn = make_float2(fminf(mn.x, x.x), fminf(mn.y, x.y));
+        }
+        *reinterpret_cast<float2*>(s_mx + st * ext_pitch + dim) = mx;
+        *reinterpret_cast<float2*>(s_mn + st * ext_pitch + dim) = mn;
+    }
+    __syncthreads();
+    // each token group's thresholds, in its first stripe's place
+    const int spg = tg / kRowsStripe, groups = (n + tg - 1) / tg;
+    for (int i = tid; i < groups * d; i += nt) {
+        const int first = i / d * spg, last = min(first + spg, stripes), dim = i % d;
+        float mx = s_mx[first * ext_pitch + dim], mn = s_mn[first * ext_pitch + dim];
+        for (int st = first + 1; st < last; ++st) {
+            mx = fmaxf(mx, s_mx[st * ext_pitch + dim]);
+            mn = fminf(mn, s_mn[st * ext_pitch + dim]);
+        }
+        s_mx[first * ext_pitch + dim] = mx * 0.5f;
+        s_mn[first * ext_pitch + dim] = mn * 0.5f;
+    }
+    __syncthreads();
+
+    for (int i = tid; i < d / CH * kRowsBlock; i += nt) {
+        const int t = i % kRowsBlock, c0 = i / kRowsBlock * CH;
+        if (t >= n) continue;
+        const int ext = t / tg * spg * ext_pitch;
+        uint32_t sw[CH / 32], mw[CH / 32];
+        float lows[CH / G], deltas[CH / G];
+        encode_chunk<T, G, true>(reinterpret_cast<const T*>(lds + t * pitch), c0, d, s_mx + ext, s_mn + ext, sw, mw,
+                                 lows, deltas);
+#pragma unroll
+        for (int wi = 0; wi < CH / 32; ++wi) {
+            s_sign[t * w + c0 / 32 + wi] = sw[wi];
+            s_mag[t * w + c0 / 32 + wi] = mw[wi];
+        }
+#pragma unroll
+        for (int rr = 0; rr < CH / G; ++rr) {
+            s_low[t * r + c0 / G + rr] = f16_rne(lows[rr]);
+            s_delta[t * r + c0 / G + rr] = f16_rne(deltas[rr]);
+        }
+    }
+    __syncthreads();
+    const int64_t orow = kvh * cap + offset + gs;
+    for (int i = tid; i < n * w; i += nt) {
+        k_sign[orow * w + i] = static_cast<int32_t>(s_sign[i]);
+        k_mag[orow * w + i] = static_cast<int32_t>(s_mag[i]);
+    }
+    for (int i = tid; i < n * r; i += nt) {
+        k_low[orow * r + i] = s_low[i];
+        k_delta[orow * r + i] = s_delta[i];
+    }
+}
+
 // Prefix prepack (APPEND false): block (x, y) encodes token group x of KV
 // head y, rows [x*tg, min(x*tg + tg, tokens)) of `keys`, into packed rows
 // y*cap + offset + x*tg + t, for the group sizes pack128_block does not
@@ -306,7 +431,17 @@ hipError_t launch_pack_t(const T* keys, int64_t kvh, int64_t tokens, int d, int6
     else if (fast)
         hipLaunchKernelGGL((pack128_kernel<T, G, false>), grid, dim3(kWave * pack128_waves<G>()), 0, stream, keys,
                            head_stride, tokens, tg, ks, km, kl, kd, cap, off, AppendArgs<T>{});
-    else
+    else if (d % (G > 32 ? G : 32) == 0 && tg % kRowsStripe == 0 && tg <= kRowsBlock &&
+             pack_rows_lds(d, G, sizeof(T)) <= kMaxStaticLds && reinterpret_cast<uintptr_t>(keys) % 16 == 0 &&
+             (head_stride * static_cast<int64_t>(sizeof(T))) % 16 == 0) {
+        // whole chunks, whole stripes and 16-byte rows that fit LDS; the rest
+        // (partial words, other groups, fp32 rows of 192 dimensions and more) keeps
+        // the general kernel
+        const int rpb = kRowsBlock / tg * tg, items = d / (G > 32 ? G : 32) * kRowsBlock;
+        hipLaunchKernelGGL((pack_rows_kernel<T, G>), dim3(static_cast<unsigned>((tokens + rpb - 1) / rpb), grid.y),
+                           dim3(items < kPackThreads ? items : kPackThreads), pack_rows_lds(d, G, sizeof(T)), stream,
+                           keys, head_stride, tokens, d, tg, rpb, ks, km, kl, kd, cap, off);
+    } else
         hipLaunchKernelGGL((pack_kernel<T, G, false>), grid, dim3(kPackThreads), 0, stream, keys, head_stride,
                            tokens, d, tg, ks, km, kl, kd, cap, off);
     return hipGetLastError();

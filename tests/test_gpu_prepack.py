@@ -33,3 +33,34 @@ def test_pack_row_blocks_bit_exact(tg, g, dtype):
         want = core.pack_keys(keys.float().numpy(), token_group_size=tg, dim_group_size=g)
         for got, expected in zip(packed, want):
             assert np.array_equal(_bits(got)[:, :tokens], expected), (tokens, got.dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("dim,tg,g", [(32, 8, 16), (64, 32, 32), (64, 24, 32), (64, 64, 64), (64, 8, 16), (96, 32, 16),
+                                      (96, 64, 32), (160, 40, 32), (192, 64, 64), (256, 16, 16), (256, 64, 32)])
+def test_pack_rows_of_other_head_sizes_bit_exact(dim, tg, g, dtype):
+    """Row blocks of head sizes other than 128 (fp32 rows of 192 and 256 dimensions
+    do not fit them): one row, the edges of stripes, groups and blocks, an
+    offset into a larger cache, the largest values and zeros of both
+    signs in the keys; exact."""
+    rows = 64 // tg * tg
+    for tokens in (1, 7, 9, rows - 1, rows, rows + 1, 2 * rows + tg + 1):
+        gen = torch.Generator().manual_seed(tokens + tg + g + dim)
+        keys = torch.randn(3, tokens, dim, generator=gen)
+        keys[:, ::5, 3] *= 10.0
+        keys[:, ::3, 5] = 0.0
+        keys[:, 1::3, 5] = -0.0
+        keys[1, tokens // 2, 7] = torch.finfo(dtype).max
+        keys[2, tokens // 2, 9] = -torch.finfo(dtype).max
+        keys = keys.to(dtype)
+        cap, offset = tokens + 2 * tg + 3, 2 * tg
+        packed = popkv_cuda.pack_keys(torch.zeros(3, cap, dim, dtype=dtype, device=DEV), token_group_size=tg,
+                                      dim_group_size=g)
+        before = [_bits(p) for p in packed]
+        popkv_cuda.pack_keys_into(keys.to(DEV), packed, token_offset=offset, token_group_size=tg, dim_group_size=g)
+        want = core.pack_keys(keys.float().numpy(), token_group_size=tg, dim_group_size=g)
+        for got, expected, old in zip(packed, want, before):
+            bits = _bits(got)
+            assert np.array_equal(bits[:, offset:offset + tokens], expected), (tokens, got.dtype)
+            assert np.array_equal(bits[:, :offset], old[:, :offset])
+            assert np.array_equal(bits[:, offset + tokens:], old[:, offset + tokens:])
