@@ -117,10 +117,35 @@ def pointer_array(pointers: list[int]) -> ctypes.Array:
     return (_vp * len(pointers))(*pointers)
 
 
-def stream_of(device: torch.device) -> int:
+def stream_of(device: torch.device | str | int) -> int:
     """hipStream_t of torch's current stream on `device`, as an integer."""
-    return torch.cuda.current_stream(device).cuda_stream
+    # without a torch.cuda.Stream object around it: a decode loop of separate
+    # operations is bound by the host, and asks for the stream at every call
+    if not isinstance(device, torch.device) or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _Current:
+    """The guard of a device that is current already: nothing to switch."""
+
+    def __enter__(self) -> None:
+        return None
+
+    def __exit__(self, *exc) -> None:
+        return None
+
+
+_CURRENT = _Current()
+
+
+def on_device(device: torch.device):
+    """torch.cuda.device(device), free of its two device exchanges where
+    `device` is current (the common case of one process per GPU)."""
+    return _CURRENT if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    status = getattr(lib(), name)(*args)
+    if status != POPKV_OK:
+        check(status)

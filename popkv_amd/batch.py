@@ -167,7 +167,7 @@ def prepack_batched(cache: BatchedPopKVCache, lengths: SequenceLengths) -> None:
         raise RuntimeError("Pop-KV cache capacity exceeded")
     dev = cache.key_cache.device
     _check_on_device(cache, lengths)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         stream = nat.stream_of(dev)
         if len(set(lengths.host)) == 1 and lengths.host[0] > 0:
             # equal lengths: one launch, the batch's B*KVH heads side by side
@@ -213,7 +213,7 @@ def append_batched(cache: BatchedPopKVCache, lengths: SequenceLengths, new_k: to
     dev = cache.key_cache.device
     _check_on_device(cache, lengths, nk, nv, status)
     ks, km, kl, kd = cache.packed
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         nat.call("popkv_append", nk.data_ptr(), nv.data_ptr(), nat.dtype_code(nk), cache.key_cache.data_ptr(),
                  cache.value_cache.data_ptr(), cache.capacity, ks.data_ptr(), km.data_ptr(), kl.data_ptr(),
                  kd.data_ptr(), int(ks.shape[2]), lengths.device.data_ptr(), batch, kv_heads, cache.group_size,
@@ -285,7 +285,7 @@ def popkv_layer_step_batched(q: torch.Tensor, cache: BatchedPopKVCache, lengths:
     kk = min(budget - 1, bound)
     idx = torch.full((batch, q_heads, kk + 1), -1, device=dev, dtype=torch.int64) if return_indices else None
     ks, km, kl, kd = cache.packed
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         if append:
             nat.call("popkv_decode_layer_batched", qc.data_ptr(), nat.dtype_code(qc), ks.data_ptr(), km.data_ptr(),
                      kl.data_ptr(), kd.data_ptr(), int(ks.shape[2]), cache.key_cache.data_ptr(),

@@ -213,7 +213,7 @@ def _stage_append(items: list[tuple[PopKVCache, torch.Tensor]]) -> bool:
             column.append(p)
     if any(len(set(column)) != len(items) for column in columns[2:]) or len({id(cache) for cache, _ in items}) != len(items):
         return False
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         staged = torch.empty((len(items), kv_heads, n + 1, 128), device=dev, dtype=dtype).unbind(0)
         active, new_k, *planes = columns
         nat.call("popkv_stage_append", *map(nat.pointer_array, (active, new_k, [t.data_ptr() for t in staged], *planes)),
@@ -449,7 +449,7 @@ def popkv_layer_step(
     kk = min(budget - 1, tokens)
     idx = torch.empty((q_heads, kk + 1), device=dev, dtype=torch.int64) if return_indices else None
     k_sign, k_mag, k_low, k_delta = cache.packed
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         nat.call("popkv_layer_step", qc.data_ptr(), nat.dtype_code(qc), k_sign.data_ptr(), k_mag.data_ptr(),
                  k_low.data_ptr(), k_delta.data_ptr(), int(k_sign.shape[1]), prefix_k.data_ptr(), prefix_v.data_ptr(),
                  prefix_k.stride(0), prefix_v.stride(0), kc.data_ptr(), vc.data_ptr(), mapping.data_ptr(), q_heads,
@@ -490,7 +490,7 @@ def popkv_layer_step_attention(q: torch.Tensor, prefix_k: torch.Tensor, prefix_v
         raise RuntimeError("popkv_layer_step_attention: every tensor must be on the same CUDA device")
     dev = q.device
     mapping = head_to_kv.to(device=dev, dtype=torch.int64).contiguous()
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         nat.call("popkv_layer_step_attention", q.data_ptr(), nat.dtype_code(q), prefix_k.data_ptr(),
                  prefix_v.data_ptr(), prefix_k.stride(0), prefix_v.stride(0), mapping.data_ptr(), q_heads, kv_heads,
                  tokens, int(budget), int(dim_group_size), ws.data_ptr(), ws.numel(), nat.stream_of(dev))
@@ -517,7 +517,7 @@ def dense_attention_step(q: torch.Tensor, prefix_k: torch.Tensor, prefix_v: torc
     # change of head count clears them, as for the layer step's histograms)
     ws = (workspace or LayerStepWorkspace()).get(nbytes, dev, q_heads)
     output = torch.empty_like(qc) if out is None else out
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         nat.call("popkv_dense_attention", qc.data_ptr(), nat.dtype_code(qc), prefix_k.data_ptr(), prefix_v.data_ptr(),
                  prefix_k.stride(0), prefix_v.stride(0), kc.data_ptr(), vc.data_ptr(), q_heads, kv_heads, tokens,
                  output.data_ptr(), ws.data_ptr(), ws.numel(), nat.stream_of(dev))

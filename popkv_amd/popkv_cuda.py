@@ -84,7 +84,7 @@ def _launch_pack(keys: torch.Tensor, packed, token_offset: int, token_group_size
                  dim_group_size: int) -> None:
     k_sign, k_mag, k_low, k_delta = packed
     kv_heads, tokens, head_dim = (int(x) for x in keys.shape)
-    with torch.cuda.device(keys.device):
+    with nat.on_device(keys.device):
         nat.call("popkv_pack", keys.data_ptr(), nat.dtype_code(keys), kv_heads, tokens, head_dim,
                  tokens * head_dim, k_sign.data_ptr(), k_mag.data_ptr(), k_low.data_ptr(), k_delta.data_ptr(),
                  int(k_sign.shape[1]), int(token_offset), token_group_size, dim_group_size,
@@ -194,7 +194,7 @@ def query_encode(queries: torch.Tensor, *, out=None, dim_group_size: int = 32):
            and tuple(q_low.shape) == rep_expected and tuple(q_delta.shape) == rep_expected,
            "query encoding outputs have incorrect shape")
     _check(all(t.device == queries.device for t in outputs), "query encoding tensors must share a CUDA device")
-    with torch.cuda.device(queries.device):
+    with nat.on_device(queries.device):
         nat.call("popkv_query_encode", queries.data_ptr(), nat.dtype_code(queries), batch * q_heads, head_dim,
                  dim_group_size, nat.ENCODE_FOLD, q_sign.data_ptr(), q_mag.data_ptr(), q_low.data_ptr(),
                  q_delta.data_ptr(), nat.stream_of(queries.device))
@@ -247,7 +247,7 @@ def score_encoded(
     _check(all(t.device == dev for t in (*encoded_query, *packed, head_to_kv)),
            "encoded score tensors must share a CUDA device")
     scores = torch.empty((batch, q_heads, tokens), device=dev, dtype=torch.float16)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         nat.call("popkv_score_encoded", q_sign.data_ptr(), q_mag.data_ptr(), q_low.data_ptr(), q_delta.data_ptr(),
                  k_sign.data_ptr(), k_mag.data_ptr(), k_low.data_ptr(), k_delta.data_ptr(), head_to_kv.data_ptr(),
                  batch, q_heads, kv_heads, int(k_sign.shape[1]), tokens, dim_group_size, scores.data_ptr(),
@@ -289,7 +289,7 @@ def score(
     scores = torch.empty((batch, q_heads, tokens), device=dev, dtype=out_dtype)
     ws_bytes = int(nat.lib().popkv_score_workspace_bytes(batch, q_heads, head_dim, dim_group_size))
     workspace = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         nat.call("popkv_score", queries.data_ptr(), nat.dtype_code(queries), batch, q_heads, head_dim,
                  k_sign.data_ptr(), k_mag.data_ptr(), k_low.data_ptr(), k_delta.data_ptr(), head_to_kv.data_ptr(),
                  kv_heads, capacity, tokens, dim_group_size, scores.data_ptr(), workspace.data_ptr(), ws_bytes,

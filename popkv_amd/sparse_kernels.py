@@ -67,7 +67,7 @@ def indexed_attention_split_partial(
     idx = idx.contiguous()
     vm = None if valid_mask is None else valid_mask.contiguous().to(torch.bool).view(torch.uint8)
     mapping = head_to_kv.to(device=queries.device, dtype=torch.int64).contiguous()
-    with torch.cuda.device(queries.device):
+    with nat.on_device(queries.device):
         nat.call("popkv_sparse_attention_partial", q.data_ptr(), nat.dtype_code(q), pk.data_ptr(), pv.data_ptr(),
                  pk.stride(0), pk.stride(1), pv.stride(0), pv.stride(1), prefix_tokens, ck.data_ptr(), cv.data_ptr(),
                  idx.data_ptr(), _INDEX_CODES[idx.dtype], nat.ptr(vm), mapping.data_ptr(), q_heads, kv_heads,
@@ -90,7 +90,7 @@ def indexed_attention_split_merge(
         raise ValueError("partial/output shape mismatch")
     output = torch.empty(output_like.shape, device=output_like.device, dtype=output_like.dtype)
     p = partials.contiguous()
-    with torch.cuda.device(output.device):
+    with nat.on_device(output.device):
         nat.call("popkv_sparse_attention_merge", p.data_ptr(), q_heads, num_splits, head_dim, output.data_ptr(),
                  nat.dtype_code(output), nat.stream_of(output.device))
     return output

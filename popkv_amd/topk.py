@@ -40,7 +40,7 @@ def _workspace(device: torch.device, stream: int, nbytes: int, rows: int) -> tor
 
 def _launch(scores2d: torch.Tensor, k: int, current: int, out: torch.Tensor) -> None:
     rows, tokens = (int(x) for x in scores2d.shape)
-    with torch.cuda.device(scores2d.device):
+    with nat.on_device(scores2d.device):
         stream = nat.stream_of(scores2d.device)
         nbytes = int(nat.lib().popkv_topk_select_workspace_bytes(rows, tokens))
         ws = _workspace(scores2d.device, int(stream or 0), nbytes, rows)
