@@ -64,10 +64,14 @@ __device__ __forceinline__ void dense_merge(const float* __restrict__ ps, int ns
             if (s0 + b > 0) load_acc(s0 + b);
 #pragma unroll
             for (int j = 0; j < NF; ++j) {
-                // (past nsplit the lane's weight is 0: m = -inf there)
-                const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), b + j));
+                // past nsplit a[j] repeats the last split, which may hold an
+                // infinity: not folded, not even with weight 0
+                if (s0 + b + j < nsplit) {
+                    const float ws =
+                        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), b + j));
 #pragma unroll
-                for (int i = 0; i < DPL; ++i) num[i] = fmaf(ws, a[j][i], num[i]);
+                    for (int i = 0; i < DPL; ++i) num[i] = fmaf(ws, a[j][i], num[i]);
+                }
             }
         }
     }

@@ -50,3 +50,35 @@ def test_dense_attention_tile_and_split_edges(kv_heads, tokens, group, dtype):
         got = popkv.dense_attention_step(q.to(DEV), pk, pv, k.to(DEV), v.to(DEV), workspace=ws)
         err = (got.cpu().double() - want).abs()
         assert (err <= ULP[dtype] * want.abs() + 4e-5).all(), float((err - ULP[dtype] * want.abs()).max())
+
+
+def _attend_nonfinite(kv_heads, group, tokens, dtype, spoil):
+    """dense_attention_step after `spoil(keys, values)`, and float64: (got,
+    want).  Small queries, so that no weight of any row underflows."""
+    gen = torch.Generator().manual_seed(tokens + group)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).to(dtype)  # noqa: E731
+    q, k, v = draw(kv_heads * group, 128) * 0.1, draw(kv_heads, 128), draw(kv_heads, 128)
+    pk, pv = draw(kv_heads, tokens, 128), draw(kv_heads, tokens, 128)
+    spoil(pk, pv)
+    got = popkv.dense_attention_step(q.to(DEV), pk.to(DEV), pv.to(DEV), k.to(DEV), v.to(DEV))
+    return got.cpu().double(), _reference(q, pk, pv, k, v)
+
+
+def _same_nonfinite(got, want, dtype):
+    assert torch.equal(got.isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(got[inf], want[inf])
+    ok = want.isfinite()
+    assert ((got[ok] - want[ok]).abs() <= ULP[dtype] * want[ok].abs() + 4e-5).all()
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16, torch.float32))
+@pytest.mark.parametrize("group", (1, 2, 4, 8))
+@pytest.mark.parametrize("kv_heads,tokens", [(2, 100), (2, 1024), (1, 4240), (1, 8191), (1, 40007)])
+def test_dense_attention_infinite_value_in_the_last_split(kv_heads, tokens, group, dtype):
+    """An infinite value element in the last row: infinite in that output
+    dimension however many splits the merge folds, finite in the others."""
+    def spoil(pk, pv):
+        pv[0, -1, 3], pv[-1, -1, 77] = float("inf"), float("-inf")
+
+    _same_nonfinite(*_attend_nonfinite(kv_heads, group, tokens, dtype, spoil), dtype)
