@@ -138,19 +138,35 @@ __global__ __launch_bounds__(kAttnThreads) void attn_dense_gqa_kernel(
     SoftmaxState st[QPK];
 #pragma unroll
     for (int j = 0; j < QPK; ++j) init_state(st[j]);
-    for (int base = 0; base < n_rows; base += ROWS_PER_PASS * NB) {
+    // tail: the split's last pass, where it is not whole.  Its dead rows
+    // re-read the split's first one; their values are cleared, since a weight
+    // of 0 would make NaN of an infinite one.
+    constexpr int PASS = ROWS_PER_PASS * NB;
+    auto pass = [&](int base, bool tail) __attribute__((always_inline)) {
         Raw8<T> kr[NB], vr[NB];
         bool live[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int r = base + b * ROWS_PER_PASS + slot;
-            live[b] = r < n_rows;
+            live[b] = !tail || r < n_rows;
             const uint32_t off = static_cast<uint32_t>(live[b] ? r : 0) * (D * sizeof(T));
             kr[b].load(reinterpret_cast<const T*>(kb + off));
             vr[b].load(reinterpret_cast<const T*>(vb + off));
         }
+        if (tail) {  // uniform
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                if (!live[b]) vr[b].zero();
+        }
 #pragma unroll
         for (int j = 0; j < QPK; ++j) fold_rows<T, NB>(st[j], qr[j], kr, vr, live, scale);
+    };
+    if constexpr (QPK <= 2) {
+        int base = 0;
+        for (; base + PASS <= n_rows; base += PASS) pass(base, false);
+        if (base < n_rows) pass(base, true);
+    } else {
+        for (int base = 0; base < n_rows; base += PASS) pass(base, base + PASS > n_rows);
     }
 #pragma unroll
     for (int j = 0; j < QPK; ++j) {
@@ -233,7 +249,9 @@ __global__ __launch_bounds__(kDenseThreads) void attn_dense_mfma_kernel(
                           : make_uint4(0u, 0u, 0u, 0u);
     const char* kb = reinterpret_cast<const char*>(kc + g * k_hs + t0 * D + 8 * grp);
     const char* vb = reinterpret_cast<const char*>(vc + g * v_hs + t0 * D + 8 * col);
-    // rows past the split's end re-read the split's first row (weight 0)
+    // rows past the split's end re-read the split's first row: the fold masks
+    // their logits and clears their values (a weight of 0 would make NaN of
+    // an infinite one)
     auto load_tile = [&](int r0, uint4 (&kt)[4], uint4 (&vt)[4]) {
         const int rk = r0 + col;
         const uint32_t ko = static_cast<uint32_t>(rk < n_rows ? rk : 0) * (D * sizeof(T));
@@ -257,7 +275,12 @@ __global__ __launch_bounds__(kDenseThreads) void attn_dense_mfma_kernel(
     for (int j = 0; j < QPK; ++j)
 #pragma unroll
         for (int d = 0; d < 8; ++d) acc[j][d] = 0.0f;
-    auto fold_tile = [&](int r0, const uint4 (&kt)[4], const uint4 (&vt)[4]) {
+    auto fold_tile = [&](int r0, const uint4 (&kt)[4], uint4 (&vt)[4]) {
+        if (r0 + TILE > n_rows) {  // uniform: the split's last tile
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (r0 + 4 * grp + r >= n_rows) vt[r] = make_uint4(0u, 0u, 0u, 0u);
+        }
         mfma_f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) c = mfma_16x16x32<T>(qa[i], kt[i], c);

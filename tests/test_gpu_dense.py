@@ -82,3 +82,17 @@ def test_dense_attention_infinite_value_in_the_last_split(kv_heads, tokens, grou
         pv[0, -1, 3], pv[-1, -1, 77] = float("inf"), float("-inf")
 
     _same_nonfinite(*_attend_nonfinite(kv_heads, group, tokens, dtype, spoil), dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16, torch.float32))
+@pytest.mark.parametrize("group", (1, 2, 4, 8))
+@pytest.mark.parametrize("kv_heads,tokens", [(2, 1), (2, 1000), (3, 2001), (1, 40007), (300, 200)])
+def test_dense_attention_infinite_value_at_a_splits_first_row(kv_heads, tokens, group, dtype):
+    """Infinite value elements in every row a split can start at (multiples
+    of 16, dimension row / 16): a pass that reaches past its split's end has
+    no live row to take there, and must not fold another's value."""
+    def spoil(pk, pv):
+        rows = torch.arange(0, tokens, 16)
+        pv[:, rows, rows // 16 % 96] = float("inf")
+
+    _same_nonfinite(*_attend_nonfinite(kv_heads, group, tokens, dtype, spoil), dtype)
