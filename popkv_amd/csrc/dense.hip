@@ -296,7 +296,9 @@ __global__ __launch_bounds__(kDenseThreads) void attn_dense_mfma_kernel(
             mx = fmaxf(mx, dpp_mov<0x140>(mx));
             const float mn = fmaxf(m_run[j], mx);
             alpha[j] = mn == -INFINITY ? 1.0f : __expf(m_run[j] - mn);  // m_run = -inf gives 0
-            p[j] = mn == -INFINITY ? 0.0f : __expf(sj - mn);           // dead rows give 0
+            // dead rows and logits of -inf give 0; a NaN logit stays NaN, also
+            // where no logit of the wave has been a number yet (mn = -inf)
+            p[j] = sj == -INFINITY ? 0.0f : __expf(sj - mn);
             moved = moved || mn != m_run[j];
             m_run[j] = mn;
             lsum[j] = fmaf(lsum[j], alpha[j], p[j]);

@@ -96,3 +96,16 @@ def test_dense_attention_infinite_value_at_a_splits_first_row(kv_heads, tokens, 
         pv[:, rows, rows // 16 % 96] = float("inf")
 
     _same_nonfinite(*_attend_nonfinite(kv_heads, group, tokens, dtype, spoil), dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16, torch.float32))
+@pytest.mark.parametrize("group", (1, 2, 4, 8))
+@pytest.mark.parametrize("first,tokens", [(0, 300), (112, 300), (288, 300), (0, 2049)])
+def test_dense_attention_tile_of_nan_keys(first, tokens, group, dtype):
+    """NaN keys in 16 rows of the second KV head that make up one tile of the
+    matrix-core kernel, the first a wave folds: NaN in every output of that
+    head's group, none elsewhere."""
+    def spoil(pk, pv):
+        pk[1, first:first + 16] = float("nan")
+
+    _same_nonfinite(*_attend_nonfinite(2, group, tokens, dtype, spoil), dtype)
