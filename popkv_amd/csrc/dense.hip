@@ -12,103 +12,152 @@
 namespace popkv {
 namespace {
 
-// Merge of one head's `nsplit` states (m, l, acc[128]) and the current token
-// by one wave, DPL dims per lane from d0 on (2: dims lane and lane + 64; 1:
-// dim d0 + lane).  The states come from other workgroups of this launch
-// (device-coherent loads), NF of them in flight at once.
-template <typename T, int DPL, int NF>
-__device__ __forceinline__ void dense_merge(const float* __restrict__ ps, int nsplit, const T* __restrict__ qh,
+// Merge of `n` <= 64 states (m, l, acc[128]) of one head, `step` states
+// apart, by one wave; DPL dims per lane from d0 on (2: dims lane and lane +
+// 64; 1: dim d0 + lane).  The states come from other workgroups of this
+// launch (device-coherent loads), NF of them in flight at once.  LAST: with
+// the current token's logit and value, num / den being the head's output;
+// else (mx, den, num) is their state.
+template <typename T, int DPL, bool LAST>
+__device__ __forceinline__ void dense_merge(const float* __restrict__ ps, int step, int n, const T* __restrict__ qh,
                                             const T* __restrict__ ck, const T* __restrict__ cv, float scale, int d0,
-                                            T* __restrict__ outh) {
-    constexpr int S = 128 + 2;
-    static_assert(kWave % NF == 0, "a batch's weights sit in one set of 64 splits");
+                                            float& mx, float& den, float (&num)[DPL]) {
+    constexpr int S = 128 + 2, NF = 32;
     const int lane = threadIdx.x & (kWave - 1);
-    const float q0 = Elem<T>::load(qh, lane), q1 = Elem<T>::load(qh, lane + 64);
-    const float k0 = Elem<T>::load(ck, lane), k1 = Elem<T>::load(ck, lane + 64);
-    float num[DPL], v[DPL];
+    float q0 = 0.0f, q1 = 0.0f, k0 = 0.0f, k1 = 0.0f, v[DPL];
+    if constexpr (LAST) {
+        q0 = Elem<T>::load(qh, lane), q1 = Elem<T>::load(qh, lane + 64);
+        k0 = Elem<T>::load(ck, lane), k1 = Elem<T>::load(ck, lane + 64);
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) v[i] = Elem<T>::load(cv, d0 + lane + 64 * i);
-    // split s0 + lane's maximum and denominator, and NF splits' accumulators
-    float m = -INFINITY, l = 0.0f, a[NF][DPL];
-    auto load_ml = [&](int s0) {
-        m = -INFINITY;
-        l = 0.0f;
-        if (s0 + lane < nsplit) {
-            m = ld_f32<true>(ps + static_cast<int64_t>(s0 + lane) * S);
-            l = ld_f32<true>(ps + (static_cast<int64_t>(s0 + lane) * S + 1));
-        }
-    };
-    auto load_acc = [&](int s0) {
+        for (int i = 0; i < DPL; ++i) v[i] = Elem<T>::load(cv, d0 + lane + 64 * i);
+    }
+    float m = -INFINITY, l = 0.0f, a[NF][DPL];  // m, l: state `lane`'s
+    if (lane < n) {
+        m = ld_f32<true>(ps + static_cast<int64_t>(lane * step) * S);
+        l = ld_f32<true>(ps + (static_cast<int64_t>(lane * step) * S + 1));
+    }
+    auto load_acc = [&](int b) {
 #pragma unroll
         for (int j = 0; j < NF; ++j) {
-            const float* src = ps + (static_cast<int64_t>(min(s0 + j, nsplit - 1)) * S + 2 + d0 + lane);
+            const float* src = ps + (static_cast<int64_t>(min(b + j, n - 1) * step) * S + 2 + d0 + lane);
 #pragma unroll
             for (int i = 0; i < DPL; ++i) a[j][i] = ld_f32<true>(src + 64 * i);
         }
     };
-    load_ml(0);
     load_acc(0);
-    float mx = m;
-    for (int s = kWave + lane; s < nsplit; s += kWave) mx = fmaxf(mx, ld_f32<true>(ps + static_cast<int64_t>(s) * S));
-    const float cur_m = wave_sum(q0 * k0 + q1 * k1) * scale;
-    mx = fmaxf(wave_max(mx), cur_m);
-    const float wc = __expf(cur_m - mx);
-    float den = 0.0f;
+    mx = wave_max(m);
+    float wc = 0.0f;
+    if constexpr (LAST) {
+        const float cur_m = wave_sum(q0 * k0 + q1 * k1) * scale;
+        mx = fmaxf(mx, cur_m);
+        wc = __expf(cur_m - mx);
+    }
+    const float w = m == -INFINITY ? 0.0f : __expf(m - mx);
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) num[i] = wc * v[i];
-    for (int s0 = 0; s0 < nsplit; s0 += kWave) {
-        if (s0 > 0) load_ml(s0);
-        const float w = m == -INFINITY ? 0.0f : __expf(m - mx);
-        den += l * w;
-        for (int b = 0; b < kWave && s0 + b < nsplit; b += NF) {
-            if (s0 + b > 0) load_acc(s0 + b);
+    for (int i = 0; i < DPL; ++i) num[i] = LAST ? wc * v[i] : 0.0f;
+    for (int b = 0; b < n; b += NF) {
+        if (b > 0) load_acc(b);
+        auto fold = [&](int j) {
+            const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), b + j));
 #pragma unroll
-            for (int j = 0; j < NF; ++j) {
-                // past nsplit a[j] repeats the last split, which may hold an
-                // infinity: not folded, not even with weight 0
-                if (s0 + b + j < nsplit) {
-                    const float ws =
-                        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), b + j));
+            for (int i = 0; i < DPL; ++i) num[i] = fmaf(ws, a[j][i], num[i]);
+        };
+        // past n a[j] repeats the last state, which may hold an infinity: not
+        // folded, not even with weight 0
 #pragma unroll
-                    for (int i = 0; i < DPL; ++i) num[i] = fmaf(ws, a[j][i], num[i]);
-                }
+        for (int j0 = 0; j0 < NF; j0 += 8) {
+            if (b + j0 + 8 <= n) {
+#pragma unroll
+                for (int j = j0; j < j0 + 8; ++j) fold(j);
+            } else {
+#pragma unroll
+                for (int j = j0; j < j0 + 8; ++j)
+                    if (b + j < n) fold(j);
             }
         }
     }
-    den = wave_sum(den) + wc;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) Elem<T>::store(outh, d0 + lane + 64 * i, num[i] / den);
+    den = wave_sum(l * w) + wc;
 }
 
 // The fused merge, as in the layer step's select + attention kernel: the
 // states went out with device-coherent stores; once this block's are
 // acknowledged (the gfx942 / gfx950 rule stated at st_f32) it takes a ticket
-// on tickets[g] (zero between calls), and the group's last block merges each
-// of its heads and resets the ticket.  WAVES waves for QPK heads: a head
-// takes one wave, or two (64 dims each) where there are enough.
+// of its KV head (zero between calls, reset by the last taker), and the last
+// block merges each of the group's heads (WAVES waves for QPK heads: a head
+// takes one wave, or two of 64 dims each where there are enough).
+//
+// One block's bursts of coherent loads, each a memory latency, add up with
+// the splits that few KV heads give (up to 256), so more than 64 splits merge
+// in two levels: the last block of every set of 32 leaves the set's merged
+// state in the place of its first one, and the last of the sets' blocks merges
+// those.  Up to 64, two bursts cost less than the second hand-off.  Layer at
+// 65536 tokens bf16, one level -> two: 1 KV head of 1 / 4 / 8 query heads
+// (256 splits) 19.8 -> 13.9, 24.9 -> 17.0, 33.2 -> 19.9 us, 2 of 4 (128) 22.8
+// -> 20.7; at 16384 tokens 4 of 4 (64) it took 17.1 against 15.7.
+// Tickets: one per KV head; in two levels one per set and one for the sets, at
+// most 12 for the 1 to 3 KV heads that give more than 64 splits (the region
+// holds 64 at least).
+constexpr int kDenseOneLevel = 64, kDenseSet = 32;
+
 template <typename T, int QPK, int WAVES>
-__device__ __forceinline__ void dense_finish(int g, const float* partials, int nsplit, uint32_t* tickets,
+__device__ __forceinline__ void dense_finish(int g, int s, float* partials, int nsplit, uint32_t* tickets,
                                              const T* q, const T* cur_k, const T* cur_v, float scale, T* out) {
-    constexpr int D = 128;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    __shared__ uint32_t s_last;
-    if (threadIdx.x == 0) {
-        const uint32_t old = __hip_atomic_fetch_add(&tickets[g], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = old + 1u == static_cast<uint32_t>(nsplit) ? 1u : 0u;
-    }
-    __syncthreads();
-    if (s_last == 0u) return;
-    if (threadIdx.x == 0) __hip_atomic_store(&tickets[g], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr int D = 128, S = D + 2;
     constexpr int DPL = 2 * QPK <= WAVES ? 1 : 2, WPH = 2 / DPL;  // dims per lane, waves per head
-    constexpr int NF = 32;
+    constexpr int UNITS = QPK * WPH;                               // waves' worth of merging
+    const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    for (int u = wave; u < QPK * WPH; u += WAVES) {
-        const int h = g * QPK + u / WPH;
-        dense_merge<T, DPL, NF>(partials + static_cast<int64_t>(h) * nsplit * (D + 2), nsplit,
-                                q + static_cast<int64_t>(h) * D, cur_k + static_cast<int64_t>(g) * D,
-                                cur_v + static_cast<int64_t>(g) * D, scale, 64 * (u % WPH),
-                                out + static_cast<int64_t>(h) * D);
+    __shared__ uint32_t s_last;
+    // whether this block is the last of `n` to come here
+    auto last_of = [&](uint32_t* ticket, int n) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t old = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_last = old + 1u == static_cast<uint32_t>(n) ? 1u : 0u;
+            if (s_last != 0u) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        return s_last != 0u;
+    };
+    auto state = [&](int h, int split) { return partials + (static_cast<int64_t>(h) * nsplit + split) * S; };
+    float mx, den, num[DPL];
+    int n = nsplit, step = 1;
+    if (nsplit <= kDenseOneLevel) {
+        if (!last_of(tickets + g, n)) return;
+    } else {
+        const int sets = (nsplit + kDenseSet - 1) / kDenseSet, set = s / kDenseSet, first = set * kDenseSet;
+        uint32_t* tk = tickets + g * (sets + 1);
+        n = min(kDenseSet, nsplit - first);
+        if (!last_of(tk + set, n)) return;
+        for (int u0 = 0; u0 < UNITS; u0 += WAVES) {
+            const int u = u0 + wave, d0 = 64 * (u % WPH);
+            float* dst = state(g * QPK + u / WPH, first);
+            if (u < UNITS) dense_merge<T, DPL, false>(dst, 1, n, q, cur_k, cur_v, scale, d0, mx, den, num);
+            // a head's two waves read the same m and l: both are past their
+            // loads before either stores
+            if constexpr (WPH == 2) __syncthreads();
+            if (u < UNITS) {
+                if (d0 == 0 && lane == 0) {
+                    st_f32<true>(dst, mx);
+                    st_f32<true>(dst + 1, den);
+                }
+#pragma unroll
+                for (int i = 0; i < DPL; ++i) st_f32<true>(dst + 2 + d0 + lane + 64 * i, num[i]);
+            }
+        }
+        n = sets;
+        step = kDenseSet;
+        if (!last_of(tk + sets, n)) return;
+    }
+    for (int u = wave; u < UNITS; u += WAVES) {
+        const int h = g * QPK + u / WPH, d0 = 64 * (u % WPH);
+        dense_merge<T, DPL, true>(state(h, 0), step, n, q + static_cast<int64_t>(h) * D,
+                                  cur_k + static_cast<int64_t>(g) * D, cur_v + static_cast<int64_t>(g) * D, scale, d0,
+                                  mx, den, num);
+#pragma unroll
+        for (int i = 0; i < DPL; ++i)
+            Elem<T>::store(out + static_cast<int64_t>(h) * D, d0 + lane + 64 * i, num[i] / den);
     }
 }
 
@@ -174,7 +223,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_dense_gqa_kernel(
                            partials + (static_cast<int64_t>(g * QPK + j) * nsplit + s) * (D + 2), true);
         __syncthreads();  // store_partial's LDS is reused by the next head
     }
-    dense_finish<T, QPK, kAttnWaves>(g, partials, nsplit, tickets, q, cur_k, cur_v, scale, out);
+    dense_finish<T, QPK, kAttnWaves>(g, s, partials, nsplit, tickets, q, cur_k, cur_v, scale, out);
 }
 
 // Matrix-core form (16-bit types): per 16-token tile one v_mfma_f32_16x16x32
@@ -403,7 +452,7 @@ __global__ __launch_bounds__(kDenseThreads) void attn_dense_mfma_kernel(
             st_f32<true>(dst + 1, l);
         }
     }
-    dense_finish<T, QPK, W>(g, partials, nsplit, tickets, q, cur_k, cur_v, scale, out);
+    dense_finish<T, QPK, W>(g, s, partials, nsplit, tickets, q, cur_k, cur_v, scale, out);
 }
 
 // Splits of a dense layer: a workgroup per CU in all (a second one per CU

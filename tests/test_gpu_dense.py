@@ -109,3 +109,24 @@ def test_dense_attention_tile_of_nan_keys(first, tokens, group, dtype):
         pk[1, first:first + 16] = float("nan")
 
     _same_nonfinite(*_attend_nonfinite(2, group, tokens, dtype, spoil), dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16, torch.float32))
+@pytest.mark.parametrize("group", (1, 2, 4, 8))
+@pytest.mark.parametrize("kv_heads,tokens", [(1, 4096), (1, 4112), (1, 8192), (1, 8193), (1, 12288), (1, 32768),
+                                             (2, 16383), (3, 11000)])
+def test_dense_attention_merge_levels(kv_heads, tokens, group, dtype):
+    """32, 33 and 64 splits (one level of one and two bursts), 65, 96, 128
+    and 256, and the 77 of three KV heads (sets of 32, then the sets): float64,
+    equal bits from the same workspace again, tickets back at zero."""
+    gen = torch.Generator().manual_seed(tokens + group)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).to(dtype)  # noqa: E731
+    q, k, v = draw(kv_heads * group, 128) * 3, draw(kv_heads, 128), draw(kv_heads, 128)
+    pk, pv = draw(kv_heads, tokens, 128), draw(kv_heads, tokens, 128)
+    want = _reference(q, pk, pv, k, v)
+    ws, args = popkv.LayerStepWorkspace(), [t.to(DEV) for t in (q, pk, pv, k, v)]
+    got = popkv.dense_attention_step(*args, workspace=ws)
+    err = (got.cpu().double() - want).abs()
+    assert (err <= ULP[dtype] * want.abs() + 4e-5).all(), float((err - ULP[dtype] * want.abs()).max())
+    assert torch.equal(popkv.dense_attention_step(*args, workspace=ws), got)
+    assert not ws.buffer[:256].any()
