@@ -469,6 +469,15 @@ struct DensePlan {
 DensePlan dense_plan(int64_t tokens, int kv_heads) {
     if (tokens <= 0) return {1, kDenseLeast};
     int64_t want = kDenseBlocks / kv_heads;
+    if (want <= 1) {
+        // A workgroup per KV head can leave most CUs idle in its last round:
+        // three of a third each where those take at most 0.8 of the rounds'
+        // time (4096 tokens bf16, one and three: 144 heads 59.4 and 51.3 us,
+        // 300 147 and 118; 176, two thirds of a round either way, 70.6 and 82).
+        const int one = (kv_heads + kDenseBlocks - 1) / kDenseBlocks;
+        const int three = (3 * kv_heads + kDenseBlocks - 1) / kDenseBlocks;
+        if (5 * three <= 12 * one) want = 3;
+    }
     if (want > dense_max_splits(tokens)) want = dense_max_splits(tokens);
     if (want < 1) want = 1;
     int64_t per = ((tokens + want - 1) / want + kDenseTile - 1) / kDenseTile * kDenseTile;
