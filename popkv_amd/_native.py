@@ -11,6 +11,7 @@ call raises.
 """
 from __future__ import annotations
 
+import array
 import ctypes
 import functools
 from pathlib import Path
@@ -112,9 +113,9 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def pointer_array(pointers: list[int]) -> ctypes.Array:
-    """A host array of device pointers."""
-    return (_vp * len(pointers))(*pointers)
+def pointer_array(pointers: list[int]) -> array.array:
+    """A host array of device pointers; a call takes its buffer_info()[0]."""
+    return array.array("Q", pointers)
 
 
 def stream_of(device: torch.device | str | int) -> int:

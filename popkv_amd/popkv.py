@@ -200,24 +200,30 @@ def _stage_append(items: list[tuple[PopKVCache, torch.Tensor]]) -> bool:
         return False
     shapes = ((kv_heads, n, 128), (kv_heads, 1, 128)) + ((kv_heads, capacity, 4),) * 2 + ((kv_heads, capacity, 128 // g),) * 2
     dtypes = (dtype, dtype, torch.int32, torch.int32, torch.float16, torch.float16)
-    columns: tuple[list[int], ...] = ([], [], [], [], [], [])
+    layers, tensors = len(items), []
     for cache, key in items:
         if cache.sealed_tokens != sealed or cache.group_size != tg or cache.dim_group_size != g or len(cache.packed) != 4:
             return False
-        for t, shape, dt, column in zip((cache.active_keys, key, *cache.packed), shapes, dtypes, columns):
-            if t.shape != shape or t.dtype != dt or t.device != dev or not t.is_contiguous():
-                return False
-            p = t.data_ptr()
-            if p % 16:
-                return False
-            column.append(p)
-    if any(len(set(column)) != len(items) for column in columns[2:]) or len({id(cache) for cache, _ in items}) != len(items):
+        tensors += (cache.active_keys, key, *cache.packed)
+    # (whole lists at a time: the interpreter bounds this call, not its kernel)
+    if [t.shape for t in tensors] != [*shapes] * layers or [t.dtype for t in tensors] != [*dtypes] * layers \
+            or set(map(torch.Tensor.get_device, tensors)) != {dev.index} \
+            or not all(map(torch.Tensor.is_contiguous, tensors)):
+        return False
+    pointers = list(map(torch.Tensor.data_ptr, tensors))
+    if any(p % 16 for p in pointers):
+        return False
+    active, new_k, *planes = (pointers[i::6] for i in range(6))
+    if any(len(set(column)) != layers for column in planes) or len({id(cache) for cache, _ in items}) != layers:
         return False
     with nat.on_device(dev):
-        staged = torch.empty((len(items), kv_heads, n + 1, 128), device=dev, dtype=dtype).unbind(0)
-        active, new_k, *planes = columns
-        nat.call("popkv_stage_append", *map(nat.pointer_array, (active, new_k, [t.data_ptr() for t in staged], *planes)),
-                 len(items), nat._DTYPES[dtype], kv_heads, n, capacity, sealed, tg, g, nat.stream_of(dev))
+        # storage of each layer's own: a kept or saved active_keys holds that layer's rows alone
+        staged = [torch.empty((kv_heads, n + 1, 128), device=dev, dtype=dtype)]
+        staged += map(torch.empty_like, staged * (layers - 1))
+        arrays = [nat.pointer_array(column) for column in
+                  (active, new_k, list(map(torch.Tensor.data_ptr, staged)), *planes)]
+        nat.call("popkv_stage_append", *(array.buffer_info()[0] for array in arrays), layers, nat._DTYPES[dtype],
+                 kv_heads, n, capacity, sealed, tg, g, nat.stream_of(dev))
     for (cache, _), keys in zip(items, staged):
         cache.active_keys = keys
         cache.token_count += 1

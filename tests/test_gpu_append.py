@@ -2,6 +2,8 @@
 replaces, bit for bit, and the calls that keep to the general path."""
 from __future__ import annotations
 
+import io
+
 import pytest
 import torch
 
@@ -77,3 +79,18 @@ def test_exhausted_reserve_is_refused_as_before():
     with pytest.raises(RuntimeError, match="Pop-KV cache reserve exhausted"):
         popkv.append_retrieval_caches(popkv.RetrievalCaches("popkv-s", caches), [torch.zeros(1, 3, 1, 128, device=DEV,
                                                                                             dtype=torch.bfloat16)] * 2)
+
+
+def test_staged_keys_are_each_layers_own():
+    """A layer's staged keys keep no other layer's rows alive, and saving
+    them writes that layer's rows alone."""
+    caches = _caches(5, 61, 64, 64, torch.bfloat16)
+    new = [torch.randn(1, 3, 1, 128).bfloat16().to(DEV) for _ in range(5)]
+    for _ in range(2):
+        popkv.append_retrieval_caches(popkv.RetrievalCaches("popkv-s", caches), new)
+        for cache in caches.values():
+            keys = cache.active_keys
+            assert keys.untyped_storage().nbytes() == keys.numel() * keys.element_size()
+            saved = io.BytesIO()
+            torch.save(keys, saved)
+            assert saved.getbuffer().nbytes < 2 * keys.numel() * keys.element_size()
