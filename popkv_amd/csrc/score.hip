@@ -235,15 +235,27 @@ hipError_t launch_encode_g(const T* q, int64_t rows, int d, int g, int order, in
     }
 }
 
-// Tokens of a matrix-core scorer workgroup: whole rounds of 512 (64 per wave), so many
-// that the launch has at most about two workgroups per CU.  Kernel time with
-// 512 / 768 / 1024 / 1536 workgroups wanted (us): 8 sequences x 65535 tokens
-// G64 43.2 / 45.8 / 44.0 / 45.2 and G16 78.2 / 79.7 / 77.8 / 85.0; one of
-// 131071 G64 14.6 / 15.4 / 15.6 / 15.7 and G16 25.4 / 29.5 / 27.4 / 27.9.
-int score_span(int64_t tokens, int64_t rows, bool batched) {
+// Tokens of a matrix-core scorer workgroup: whole rounds of 512 (64 per wave),
+// so many that the launch wants this many workgroups (us, whole calls unless
+// scores are named):
+//   - 512, two per CU: 8 heads of 131071 tokens with 256 / 512 / 1024, G32 4
+//     heads a group 35.7 / 33.9 / 35.9, G64 32.3 / 30.6 / 32.0.
+//   - A batched launch 1024: the plan sees the longest sequence only, and in
+//     a ragged batch the workgroups of the short ones end at once (5
+//     sequences from 65535 tokens down to 6553, 8 heads, with 512 / 1024: G32
+//     of 8 101 / 85, G16 of 4 83 / 67; all 65535: 111 / 115 and 85 / 89).
+//   - In a layer step every workgroup adds its histogram to the row's, so
+//     few rows take fewer of them: 2 heads of 131071 tokens, 8 a group, with
+//     256 / 512: G16 30.4 / 36.0, G64 26.1 / 27.7 (popcounts 34.6 and 27.3);
+//     the same 2048 counters a workgroup beside the longest scoring (G16 groups
+//     of 8) at any row count (8 heads of 90000 tokens 48.1 / 51.4), in a batch
+//     of up to 4 rows (2 x 65535 of 2 heads, with 256 / 1024: 29.8 / 33.8).
+//     Scores alone keep 512 (G16, 4 heads a group: 7.6 / 8.0).
+int score_span(int g, int qpk, int64_t tokens, int64_t rows, bool step, bool batched) {
     constexpr int64_t kRound = kScoreThreads / kWave * kScoreGroup;
-    const int64_t kBlocks = batched ? 1024 : 512;
-    const int64_t per_row = rows < kBlocks ? kBlocks / rows : 1;
+    const bool fewer = step && (rows <= 2 || (g == 16 && qpk == 8 && (!batched || rows <= 4)));
+    const int64_t blocks = fewer ? 256 : batched ? 1024 : 512;
+    const int64_t per_row = rows < blocks ? blocks / rows : 1;
     const int64_t rounds = (tokens + kRound * per_row - 1) / (kRound * per_row);
     return static_cast<int>(rounds * kRound);
 }
@@ -304,7 +316,7 @@ hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float
         return hipGetLastError();
     }
     if (score_takes_mfma(G, qpk, batch * kvh * tokens)) {
-        const int span = score_span(tokens, batch * kvh, seq.tokens != nullptr);
+        const int span = score_span(G, qpk, tokens, batch * kvh, !std::is_void_v<QT>, seq.tokens != nullptr);
         grid.x = static_cast<unsigned>((tokens + span - 1) / span);
 #define POPKV_SCORE_MFMA(Q)                                                                                             \
     hipLaunchKernelGGL((score_d128_mfma_kernel<G, Q, QT>), grid, dim3(kScoreThreads), 0, stream, qs, qm, ql, qd, q_raw, \
