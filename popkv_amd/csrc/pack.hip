@@ -413,9 +413,12 @@ hipError_t launch_pack_t(const T* keys, int64_t kvh, int64_t tokens, int d, int6
                       (reinterpret_cast<uintptr_t>(ks) % 16 == 0) && (reinterpret_cast<uintptr_t>(km) % 16 == 0) &&
                       (reinterpret_cast<uintptr_t>(kl) % 16 == 0) && (reinterpret_cast<uintptr_t>(kd) % 16 == 0);
     constexpr bool kStageable = sizeof(T) == 2;
-    // the block form wherever the groups fill its rows: it is faster at every
-    // preset (figures at pack128_block)
-    if (fast) {
+    // the block form (figures at pack128_block), but for one group of up to 64
+    // rows (a short prefix, the append of one layer): there a workgroup is
+    // the group either way, and the block's 128-row workgroup half empty
+    // (us, block and group form, 64 tokens x 8 heads in 128-token groups: G16
+    // fp32 5.32 / 4.90, G32 fp32 5.23 / 4.62, G64 bf16 5.71 / 5.57; 100 tokens 6.0 / 6.4)
+    if (fast && (tokens > tg || tokens > 64)) {
         switch (tg) {
             case 8: return launch_pack_block<T, G, 8>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);
             case 16: return launch_pack_block<T, G, 16>(keys, kvh, tokens, head_stride, ks, km, kl, kd, cap, off, stream);

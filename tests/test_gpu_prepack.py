@@ -36,6 +36,25 @@ def test_pack_row_blocks_bit_exact(tg, g, dtype):
 
 
 @pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("tg,g", [(tg, g) for tg in (8, 16, 32, 64, 128) for g in (16, 32, 64)])
+def test_pack_of_one_group_bit_exact(tg, g, dtype):
+    """One token group, the line between its own workgroup and a row block
+    (64 rows) among its lengths, encoded in place behind two sealed groups."""
+    for tokens in sorted({1, tg // 2 + 1, min(tg, 63), min(tg, 64), min(tg, 65), tg}):
+        gen = torch.Generator().manual_seed(tokens + tg + g)
+        keys = torch.randn(3, tokens, 128, generator=gen).to(dtype)
+        cap, offset = 4 * tg, 2 * tg
+        packed = popkv_cuda.pack_keys(torch.zeros(3, cap, 128, dtype=dtype, device=DEV), token_group_size=tg,
+                                      dim_group_size=g)
+        before = [_bits(p) for p in packed]
+        popkv_cuda.pack_keys_into(keys.to(DEV), packed, token_offset=offset, token_group_size=tg, dim_group_size=g)
+        want = core.pack_keys(keys.float().numpy(), token_group_size=tg, dim_group_size=g)
+        for got, expected, old in zip(packed, want, before):
+            old[:, offset:offset + tokens] = expected
+            assert np.array_equal(_bits(got), old), (tokens, got.dtype)
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16, torch.float16))
 @pytest.mark.parametrize("dim,tg,g", [(32, 8, 16), (64, 32, 32), (64, 24, 32), (64, 64, 64), (64, 8, 16), (96, 32, 16),
                                       (96, 64, 32), (160, 40, 32), (192, 64, 64), (256, 16, 16), (256, 64, 32)])
 def test_pack_rows_of_other_head_sizes_bit_exact(dim, tg, g, dtype):
