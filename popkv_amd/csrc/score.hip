@@ -326,6 +326,7 @@ hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float
 #undef POPKV_SCORE_MFMA
         return hipGetLastError();
     }
+    // groups of 8 heads, and of 4 at G16, are the matrix cores' (score_takes_mfma)
     if constexpr (TPT == 2) {
         // fewer two-token workgroups than the chip's 256 CUs (short rows):
         // one token per thread, twice the workgroups
@@ -335,7 +336,6 @@ hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float
                 case 1: POPKV_SCORE_LAUNCH_T(1, false, 1); break;
                 case 2: POPKV_SCORE_LAUNCH_T(2, false, 1); break;
                 case 4: POPKV_SCORE_LAUNCH_T(4, false, 1); break;
-                case 8: POPKV_SCORE_LAUNCH_T(8, false, 1); break;
                 default: POPKV_SCORE_LAUNCH_T(0, false, 1); break;
             }
             return hipGetLastError();
@@ -344,8 +344,10 @@ hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float
     switch (qpk) {
         case 1: POPKV_SCORE_LAUNCH(1, false); break;
         case 2: POPKV_SCORE_LAUNCH(2, false); break;
-        case 4: POPKV_SCORE_LAUNCH(4, false); break;
-        case 8: POPKV_SCORE_LAUNCH(8, false); break;
+        case 4:
+            if constexpr (G == 16) return hipErrorInvalidValue;
+            else POPKV_SCORE_LAUNCH(4, false);
+            break;
         default: POPKV_SCORE_LAUNCH(0, false); break;
     }
 #undef POPKV_SCORE_LAUNCH
