@@ -83,13 +83,12 @@ __device__ __forceinline__ void encode_chunk(const T* __restrict__ row, int c0, 
     }
 }
 
-template <typename T, int G, bool FAST>
+template <typename T, int G>
 __global__ __launch_bounds__(kPackThreads) void pack_kernel(
-    const T* __restrict__ keys, int64_t head_stride, int64_t tokens, int d, int tg,
+    const T* __restrict__ keys, int64_t head_stride, int64_t tokens, int D, int tg,
     int32_t* __restrict__ k_sign, int32_t* __restrict__ k_mag,
     uint16_t* __restrict__ k_low, uint16_t* __restrict__ k_delta,
     int64_t cap, int64_t offset) {
-    const int D = FAST ? 128 : d;
     const int W = (D + 31) / 32;
     const int R = (D + G - 1) / G;
     const int64_t kvh = blockIdx.y;
@@ -131,54 +130,24 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
     for (int64_t t = gs + tid; t < ge; t += kPackThreads) {
         const T* row = base + t * D;
         const int64_t orow = kvh * cap + offset + t;
-        if constexpr (FAST) {
-            uint32_t sw[4], mw[4];
-            float lows[128 / G], deltas[128 / G];
+        for (int c0 = 0; c0 < D; c0 += CH) {
+            uint32_t sw[CH / 32], mw[CH / 32];
+            float lows[CH / G], deltas[CH / G];
+            encode_chunk<T, G, false>(row, c0, D, s_hi, s_lo, sw, mw, lows, deltas);
 #pragma unroll
-            for (int c = 0; c < 128 / CH; ++c)
-                encode_chunk<T, G, true>(row, c * CH, 128, s_hi, s_lo, sw + c * (CH / 32), mw + c * (CH / 32),
-                                         lows + c * (CH / G), deltas + c * (CH / G));
-            reinterpret_cast<uint4*>(k_sign)[orow] = make_uint4(sw[0], sw[1], sw[2], sw[3]);
-            reinterpret_cast<uint4*>(k_mag)[orow] = make_uint4(mw[0], mw[1], mw[2], mw[3]);
-            constexpr int RR = 128 / G;
-            uint32_t lo_p[RR / 2], de_p[RR / 2];
-#pragma unroll
-            for (int r = 0; r < RR / 2; ++r) {
-                lo_p[r] = static_cast<uint32_t>(f16_rne(lows[2 * r])) |
-                          (static_cast<uint32_t>(f16_rne(lows[2 * r + 1])) << 16);
-                de_p[r] = static_cast<uint32_t>(f16_rne(deltas[2 * r])) |
-                          (static_cast<uint32_t>(f16_rne(deltas[2 * r + 1])) << 16);
-            }
-            if constexpr (RR == 2) {
-                reinterpret_cast<uint32_t*>(k_low)[orow] = lo_p[0];
-                reinterpret_cast<uint32_t*>(k_delta)[orow] = de_p[0];
-            } else if constexpr (RR == 4) {
-                reinterpret_cast<uint2*>(k_low)[orow] = make_uint2(lo_p[0], lo_p[1]);
-                reinterpret_cast<uint2*>(k_delta)[orow] = make_uint2(de_p[0], de_p[1]);
-            } else {
-                reinterpret_cast<uint4*>(k_low)[orow] = make_uint4(lo_p[0], lo_p[1], lo_p[2], lo_p[3]);
-                reinterpret_cast<uint4*>(k_delta)[orow] = make_uint4(de_p[0], de_p[1], de_p[2], de_p[3]);
-            }
-        } else {
-            for (int c0 = 0; c0 < D; c0 += CH) {
-                uint32_t sw[CH / 32], mw[CH / 32];
-                float lows[CH / G], deltas[CH / G];
-                encode_chunk<T, G, false>(row, c0, D, s_hi, s_lo, sw, mw, lows, deltas);
-#pragma unroll
-                for (int wi = 0; wi < CH / 32; ++wi) {
-                    const int w = c0 / 32 + wi;
-                    if (w < W) {
-                        k_sign[orow * W + w] = static_cast<int32_t>(sw[wi]);
-                        k_mag[orow * W + w] = static_cast<int32_t>(mw[wi]);
-                    }
+            for (int wi = 0; wi < CH / 32; ++wi) {
+                const int w = c0 / 32 + wi;
+                if (w < W) {
+                    k_sign[orow * W + w] = static_cast<int32_t>(sw[wi]);
+                    k_mag[orow * W + w] = static_cast<int32_t>(mw[wi]);
                 }
+            }
 #pragma unroll
-                for (int rr = 0; rr < CH / G; ++rr) {
-                    const int r = c0 / G + rr;
-                    if (r < R) {
-                        k_low[orow * R + r] = f16_rne(lows[rr]);
-                        k_delta[orow * R + r] = f16_rne(deltas[rr]);
-                    }
+            for (int rr = 0; rr < CH / G; ++rr) {
+                const int r = c0 / G + rr;
+                if (r < R) {
+                    k_low[orow * R + r] = f16_rne(lows[rr]);
+                    k_delta[orow * R + r] = f16_rne(deltas[rr]);
                 }
             }
         }
@@ -445,7 +414,7 @@ hipError_t launch_pack_t(const T* keys, int64_t kvh, int64_t tokens, int d, int6
                            dim3(items < kPackThreads ? items : kPackThreads), pack_rows_lds(d, G, sizeof(T)), stream,
                            keys, head_stride, tokens, d, tg, rpb, ks, km, kl, kd, cap, off);
     } else
-        hipLaunchKernelGGL((pack_kernel<T, G, false>), grid, dim3(kPackThreads), 0, stream, keys, head_stride,
+        hipLaunchKernelGGL((pack_kernel<T, G>), grid, dim3(kPackThreads), 0, stream, keys, head_stride,
                            tokens, d, tg, ks, km, kl, kd, cap, off);
     return hipGetLastError();
 }
