@@ -49,22 +49,19 @@ def test_scores_bit_exact_at_group_and_span_edges(kv_heads, qpk, tokens, g):
     assert np.all((got[nan] & 0x7C00 == 0x7C00) & (got[nan] & 0x03FF != 0))
 
 
-@pytest.mark.parametrize("method", ("popkv-s", "popkv-q", "popkv-normal"))
-def test_ragged_batch_selects_as_the_oracle(method):
-    """Sequences from one token to several spans in one launch (spans past a
-    sequence's end return at once): the selected indices of every sequence."""
+def _ragged(method, lengths, budget, kvh, qpk):
+    """A batched layer step of `lengths` selects in every sequence what the
+    oracle does; twice, as the histograms are zero again after the first."""
     tg, g = popkv.POPKV_PRESETS[method]
-    lengths, budget, kvh, qpk = [9001, 1, 2048, 700, 4097], 256, 2, 8
     gen = torch.Generator().manual_seed(g)
-    rows = max(lengths) + 1
-    kc = torch.randn(len(lengths), kvh, rows, 128, generator=gen).half().to(DEV)
-    q = torch.randn(len(lengths), kvh * qpk, 128, generator=gen).half().to(DEV)
-    k = torch.randn(len(lengths), kvh, 128, generator=gen).half().to(DEV)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).half().to(DEV)  # noqa: E731
+    kc, q = draw(len(lengths), kvh, max(lengths) + 1, 128), draw(len(lengths), kvh * qpk, 128)
+    k = draw(len(lengths), kvh, 128)
     mapping = torch.arange(kvh * qpk, device=DEV) // qpk
     seq = pb.SequenceLengths.create(lengths, DEV)
     cache = pb.build_batched_popkv_cache(kc, kc.clone(), seq, group_size=tg, dim_group_size=g)
     ws = popkv.LayerStepWorkspace()
-    for _ in range(2):  # the histograms are zero again after the first
+    for _ in range(2):
         _, idx = pb.popkv_layer_step_batched(q, cache, seq, k, k, mapping, budget=budget, workspace=ws,
                                              return_indices=True)
     for i, n in enumerate(lengths):
@@ -73,3 +70,38 @@ def test_ragged_batch_selects_as_the_oracle(method):
         scores = core.score_encoded(enc, planes, head_to_kv=mapping.cpu().numpy(), tokens=n, dim_group_size=g)
         kk = min(budget - 1, n)
         assert np.array_equal(idx[i, :, :kk + 1].cpu().numpy(), core.select(scores[0], kk, n)), n
+
+
+@pytest.mark.parametrize("method", ("popkv-s", "popkv-q", "popkv-normal"))
+def test_ragged_batch_selects_as_the_oracle(method):
+    """Sequences from one token to several spans in one launch (spans past a
+    sequence's end return at once); a span is one round of 512 tokens here."""
+    _ragged(method, [9001, 1, 2048, 700, 4097], 256, 2, 8)
+
+
+@pytest.mark.parametrize("qpk", (4, 8))
+@pytest.mark.parametrize("method", ("popkv-q", "popkv-normal"))
+def test_ragged_batch_with_spans_of_two_rounds(method, qpk):
+    """40 rows of 20001 tokens make spans of two rounds (1024 tokens): each
+    wave's next group in flight behind its first, sequences that end in the
+    second round, in the first, at a round's and at a span's end."""
+    _ragged(method, [20001, 9400, 700, 2560, 8192], 1024, 8, qpk)
+
+
+@pytest.mark.parametrize("kv_heads,qpk,tokens,method", [(1, 8, 140001, "popkv-q"), (2, 4, 200003, "popkv-q"),
+                                                        (2, 8, 131600, "popkv-s"), (8, 8, 40001, "popkv-q"),
+                                                        (8, 4, 70001, "popkv-normal")])
+def test_step_with_spans_of_several_rounds(kv_heads, qpk, tokens, method):
+    """One layer step of few rows (256 workgroups), of G16 groups of 8 (256)
+    and of others (512): spans of 2 to 4 rounds, the last one short."""
+    tg, g = popkv.POPKV_PRESETS[method]
+    gen = torch.Generator(DEV).manual_seed(tokens)
+    draw = lambda *shape: torch.randn(*shape, generator=gen, device=DEV).half()  # noqa: E731
+    keys, q, k = draw(kv_heads, tokens, 128), draw(kv_heads * qpk, 128), draw(kv_heads, 128)
+    mapping = torch.arange(kv_heads * qpk, device=DEV) // qpk
+    cache = popkv.build_popkv_cache(keys, group_size=tg, dim_group_size=g, reserve_tokens=64)
+    _, idx = popkv.popkv_layer_step(q, cache, keys, keys, k, k, mapping, budget=2048, return_indices=True)
+    enc = core.query_encode(q[None].float().cpu().numpy(), g, order="fold")
+    planes = core.pack_keys(keys.float().cpu().numpy(), token_group_size=tg, dim_group_size=g)
+    scores = core.score_encoded(enc, planes, head_to_kv=mapping.cpu().numpy(), tokens=tokens, dim_group_size=g)
+    assert np.array_equal(idx.cpu().numpy(), core.select(scores[0], 2047, tokens))
