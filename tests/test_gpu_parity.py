@@ -642,9 +642,8 @@ def test_layer_step_batch_laid_along_heads_equals_per_sequence_steps():
 @pytest.mark.parametrize("context,dtype", [(3000, torch.bfloat16), (700, torch.float32), (1, torch.bfloat16),
                                            (1537, torch.float16), (12000, torch.bfloat16), (40000, torch.bfloat16)])
 def test_dense_attention_matches_oracle(context, dtype):
-    """The full layers: every prefix token plus the current one.  12000 and
-    40000 tokens give 24 and 79 splits of 512: the four-wave merge, with a
-    second batch round for 79."""
+    """The full layers: every prefix token plus the current one, from no
+    prefix to 32 splits (one full burst of the merge) of each KV head."""
     base = workloads.scaled(workloads.C1, context=context, budget=2)
     w = workloads.Workload(base.name, base.method, base.q_heads, base.kv_heads, 128, context, 2, base.token_group,
                            base.dim_group, dtype, 5, context > 1)
@@ -658,15 +657,15 @@ def test_dense_attention_matches_oracle(context, dtype):
     np.testing.assert_allclose(f32(out), want, atol=ATTN_ATOL, rtol=ATTN_RTOL)
 
 
-def test_dense_attention_fused_merge_tickets_and_split_limit():
-    """The MFMA dense kernel's fused merge (each KV group's last workgroup
-    merges; tickets zero between calls): one reused workspace, calls at 64
-    splits (32768 tokens: fused), 65 splits (the separate merge), 8 query
-    heads and again 32 (the ticket region cleared on the head-count change),
-    each against the oracle; and the same call twice gives equal bits."""
+def test_dense_attention_merge_tickets_and_split_limit():
+    """The merge inside the dense launch (tickets zero between calls): one
+    reused workspace, 32 splits of 8 KV heads, 33 and 64 of 4 and 65 of 3 (one
+    burst, two, and the first count of two levels), 8 query heads, and 32
+    again (the ticket region cleared on the head-count change), each against the
+    oracle; and the same call twice gives equal bits."""
     ws = popkv.LayerStepWorkspace()
-    for q_heads, kv_heads, context, seed in ((32, 8, 32769, 1), (32, 8, 33281, 2), (8, 2, 5000, 3),
-                                             (32, 8, 32769, 4)):
+    for q_heads, kv_heads, context, seed in ((32, 8, 32769, 1), (32, 8, 33281, 2), (16, 4, 4225, 5), (16, 4, 32769, 6),
+                                             (12, 3, 8194, 7), (8, 2, 5000, 3), (32, 8, 32769, 4)):
         base = workloads.scaled(workloads.C1, context=context, budget=2)
         w = workloads.Workload(base.name, base.method, q_heads, kv_heads, 128, context, 2, base.token_group,
                                base.dim_group, torch.bfloat16, seed, True)
@@ -688,9 +687,9 @@ def test_dense_attention_fused_merge_tickets_and_split_limit():
                                                      (16, 2, torch.bfloat16), (8, 2, torch.float16),
                                                      (16, 4, torch.float32)])
 def test_dense_attention_group_sizes(q_heads, kv_heads, dtype):
-    """Dense layers at every GQA group size the launcher distinguishes: 1, 2
-    and 8 query heads per KV head (VALU kernel), 4 in fp16 (matrix-core
-    kernel) and 4 in fp32 (VALU kernel); 2100 tokens end in a ragged split."""
+    """Dense layers at every GQA group size the launcher distinguishes: 1, 2,
+    4 and 8 query heads per KV head in 16-bit types (matrix-core kernel) and 4
+    in fp32 (VALU kernel); 2100 tokens end in a ragged split."""
     base = workloads.scaled(workloads.C1, context=2101, budget=2)
     w = workloads.Workload(base.name, base.method, q_heads, kv_heads, 128, 2101, 2, base.token_group,
                            base.dim_group, dtype, 9, True)
