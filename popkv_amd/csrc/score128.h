@@ -759,6 +759,12 @@ __device__ __forceinline__ void score_mfma_body(
     Group cur;
     load_group(wave, cur);
     const int64_t ntok_b = min(max(ntok_v, static_cast<int64_t>(0)), tokens);
+    // a batched step's span past its sequence's end: nothing to score, count
+    // or write (the select reads neither its keys nor its window record)
+    if (STEP && seq.tokens != nullptr &&
+        t_begin >= static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(ntok_b))))
+        return;
+
     __shared__ GroupState<G, QPK> st;
     __shared__ uint32_t s_hist[STEP ? QPK : 1][256];
     // each wave's outputs of its current group; rows 32 bytes apart modulo
@@ -769,11 +775,6 @@ __device__ __forceinline__ void score_mfma_body(
     if constexpr (STEP) {
         for (int i = threadIdx.x; i < QPK * 256; i += kScoreThreads) (&s_hist[0][0])[i] = 0u;
     }
-    // a batched step's span past its sequence's end: nothing to score, count
-    // or write (the select reads neither its keys nor its window record)
-    if (STEP && seq.tokens != nullptr &&
-        t_begin >= static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(ntok_b))))
-        return;
     if constexpr (!STEP) {
         load_group_state<G>(q_sign, q_mag, q_low, q_delta, qrow0, QPK, st);
     } else {
