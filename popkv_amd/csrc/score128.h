@@ -407,9 +407,12 @@ __device__ __forceinline__ void score_d128_body(
             for (int i = threadIdx.x; i < QPK * kWinBins * 64; i += kScoreThreads) (&s_win[0][0][0])[i] = 0u;
         }
     }
-    // a batched step's tile past its sequence's end: nothing to score, count
-    // or write (the select reads neither its keys nor its window record)
-    if (STEP && seq.tokens != nullptr &&
+    // a tile past its sequence's end in a batch: nothing to score, count or
+    // write (the select reads neither its keys nor its window record).  Not
+    // with one sequence, whose own bound is the grid's: the wait for its
+    // count costs more there (32 heads over 8 KV heads, 32767 tokens G64, the
+    // step with its append 26.7 us without it, 27.2 with)
+    if (STEP && seq.tokens != nullptr && gridDim.y > static_cast<uint32_t>(kv_heads) &&
         static_cast<int64_t>(tile) * TPT * kScoreThreads >= static_cast<int64_t>(__builtin_amdgcn_readfirstlane(
             static_cast<int>(min(max(ntok_v, static_cast<int64_t>(0)), tokens)))))
         return;
