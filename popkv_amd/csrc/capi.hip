@@ -791,8 +791,9 @@ int popkv_layer_step_attention(const void* queries, int32_t dtype, const void* p
 }
 
 // Dense-attention workspace: [align_up(QH * 4)] u32 merge tickets (zero
-// between calls; KVH <= QH of them used) | [QH][splits][130] f32 partials,
-// sized for the most splits any KV head count gives.
+// between calls; one per KV head, or at most 12 of the 64 or more where a
+// merge has two levels) | [QH][splits][130] f32 partials, sized for the most
+// splits any KV head count gives.
 size_t dense_tickets_bytes(int64_t q_heads) { return align_up(static_cast<size_t>(q_heads) * 4); }
 
 size_t popkv_dense_attention_workspace_bytes(int64_t q_heads, int64_t tokens) {

@@ -162,9 +162,12 @@ __device__ __forceinline__ void dense_finish(int g, int s, float* partials, int 
 }
 
 // VALU form (fp32; at the copy rate: 32 query heads over 8 KV heads at 32767
-// tokens 54.0 us for 268 MB, 56.5 with a merge launch): workgroup (s, g) reads each row of its split once and folds it
-// into QPK online-softmax states (one Q.K dot and one V update per head per
-// row).
+// tokens 54.2 us for 268 MB, 56.9 with a merge launch): workgroup (s, g) reads
+// each row of its split once and folds it into QPK online-softmax states (one
+// Q.K dot and one V update per head per row).  The last pass apart for 1 and
+// 2 heads, in the loop for 4 and 8 (the better one for each: 8 KV heads at
+// 65536 tokens, 2 heads 96.7 us apart and 99.7 in the loop, 8 heads 112.6 and
+// 108.7).
 template <typename T, int NB, int QPK>
 __global__ __launch_bounds__(kAttnThreads) void attn_dense_gqa_kernel(
     const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, int64_t k_hs, int64_t v_hs,
@@ -240,8 +243,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_dense_gqa_kernel(
 // each with the next tile's K and V loads in flight while it folds one.
 // Measured (HIP graph, before -> now, the whole layer): 64 query heads over 8
 // KV heads at 50001 tokens bf16 97.7 (VALU kernel and a merge launch) -> 45.9
-// us (4.5 TB/s; a copy's rate would take 40); 16 over 2 at 2000 tokens 31 ->
-// 9.5; 32 over 8 at 32767 33.8 -> 30.3; 32 over 32 at 8191 fp16 29.2 -> 27.5.
+// us (4.5 TB/s; a copy's rate would take 40); 16 over 2 at 2000 tokens 28.6 ->
+// 9.9; 32 over 8 at 32767 34.4 -> 31.2; 32 over 32 at 8191 fp16 29.1 -> 28.4.
 template <typename T> struct MfmaVec8;
 template <> struct MfmaVec8<bf16_t> { typedef __bf16 type __attribute__((ext_vector_type(8))); };
 template <> struct MfmaVec8<f16_t> { typedef _Float16 type __attribute__((ext_vector_type(8))); };

@@ -243,8 +243,8 @@ hipError_t launch_layer_step_fused(const void* queries, int dtype, const int32_t
 // Dense attention over every prefix token and the current one (head_dim 128,
 // contiguous rows; tokens may be 0) in one launch: query head h reads KV head
 // h / (QH / KVH) (group sizes 1, 2, 4, 8).  partials: q_heads *
-// dense_max_splits(tokens) states of 130 floats; tickets[KVH]: zero on entry,
-// left zero.
+// dense_max_splits(tokens) states of 130 floats; tickets: max(KVH, 64), zero
+// on entry, left zero.
 int64_t dense_max_splits(int64_t tokens);
 hipError_t launch_attention_dense(const void* queries, int dtype, const void* prefix_k, const void* prefix_v,
                                   int64_t k_head_stride, int64_t v_head_stride, int64_t tokens, int q_heads,

@@ -2,9 +2,9 @@
 //
 // head_dim 128, token groups of 8 .. 128 (powers of two): pack128_block_kernel
 // (pack128_block in pack128.h), one workgroup per 64 rows (128 for 128-token
-// groups).  Other group sizes and the append: pack128_kernel, one workgroup
-// per (KV head, token group), one wave per chunk of max(G, 32) dimensions
-// (pack128_group in pack128.h).  In both, the extrema of each dimension over
+// groups).  Other group sizes, one short group and the append: pack128_kernel,
+// one workgroup per (KV head, token group), one wave per chunk of max(G, 32)
+// dimensions (pack128_group in pack128.h).  In both, the extrema of each dimension over
 // its token group come first (thresholds 0.5*max / 0.5*min in LDS), then one
 // token per lane: the sign/magnitude words and the representatives, reduced
 // in one lane's registers in the production tree order, so the bit-exact
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_rows_kernel(
 // Prefix prepack (APPEND false): block (x, y) encodes token group x of KV
 // head y, rows [x*tg, min(x*tg + tg, tokens)) of `keys`, into packed rows
 // y*cap + offset + x*tg + t, for the group sizes pack128_block does not
-// take.  Fused append (APPEND true): block i appends
+// take and for one group of up to 64 rows.  Fused append (APPEND true): block i appends
 // the new token of (sequence, KV head) i (pack128_append).  STAGE (16-bit
 // rows; tg <= 64 at G 64, tg <= 128 at G 32 / G 16): the group's rows are
 // read from memory once, into LDS, and the encode pass reads them there.

@@ -563,7 +563,7 @@ __device__ __forceinline__ void score_d128_body(
     }
 }
 
-// ---- the matrix-core scorer (GQA groups of 4 or 8 query heads, long rows) ----
+// ---- the matrix-core scorer (GQA groups of 8 query heads, and of 4 at G16 or on long rows) ----
 //
 // The four agreement counts of a representative are inner products of small
 // integer vectors over its dimensions: with s = +-1 the sign and m in {0, 1}
@@ -666,21 +666,21 @@ __device__ __forceinline__ void wave_lds_order() {
 
 // The scorer's workgroup: tokens [t_begin, t_begin + span) of block row
 // `grow` (sequence, KV group slot; batch * kv_heads rows), span a multiple
-// of 512.  QT is the raw query
-// type when the kernel encodes the query itself (layer step), void when it
-// reads a pre-encoded state.  Wave w takes the span's groups of 64 tokens w,
-// w + 8, ..., each loaded with one 16-byte word per lane and plane a group
-// ahead of its use, spread to the operand layout by lane-row swaps, and
-// leaving through the wave's own strip of LDS in whole 16-byte words: no
-// barrier between the encode and the histogram's end.
+// of 512.  QT is the raw query type when the kernel encodes the query itself
+// (layer step), void when it reads a pre-encoded state.  Wave w takes the
+// span's groups of 64 tokens w, w + 8, ..., each loaded with one 16-byte word
+// per lane and plane a group ahead of its use, spread to the operand layout
+// by lane-row swaps, and leaving through the wave's own strip of LDS, 128
+// contiguous bytes per head and store (8 bytes a lane; 2 for scores at any
+// stride): no barrier between the encode and the histogram's end.
 //
 // The scorer streams KVH (32 + 4 R) bytes per token, so on long rows a
 // workgroup per tile would have every workgroup load at once, then all
 // compute, and pay the query's load and encode (about 2 us) per tile; here
-// the launch gives each CU two workgroups whose spans cover the rows.  Kernel
-// time before (popcounts, a workgroup per tile) -> now, 32 query heads over 8
-// KV heads: 131071 tokens G64 16.9 -> 14.6 us (3.4 TB/s of 50 MB), G16 35.4
-// -> 25.4; 8 x 65535 tokens G64 47.8 -> 43.2 us (4.6 TB/s of 201 MB).
+// spans cover the rows (how many: score_span).  Kernel time before
+// (popcounts, a workgroup per tile) -> now, 32 query heads over 8 KV heads:
+// 131071 tokens G64 16.9 -> 13.6 us (3.7 TB/s of 50 MB), 32767 tokens G16
+// 10.5 -> 8.8; 8 x 65535 tokens G64 50.7 -> 43.9 us (4.6 TB/s of 201 MB).
 template <int G, int QPK, typename QT>
 __device__ __forceinline__ void score_mfma_body(
     const int32_t* __restrict__ q_sign, const int32_t* __restrict__ q_mag,
