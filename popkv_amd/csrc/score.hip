@@ -240,7 +240,7 @@ hipError_t launch_encode_g(const T* q, int64_t rows, int d, int g, int order, in
 // scores are named):
 //   - 512, two per CU: 8 heads of 131071 tokens with 256 / 512 / 1024, G32 4
 //     heads a group 35.7 / 33.9 / 35.9, G64 32.3 / 30.6 / 32.0.
-//   - A batched launch 1024: the plan sees the longest sequence only, and in
+//   - A batch of several 1024: the plan sees the longest sequence only, and in
 //     a ragged batch the workgroups of the short ones end at once (5
 //     sequences from 65535 tokens down to 6553, 8 heads, with 512 / 1024: G32
 //     of 8 101 / 85, G16 of 4 83 / 67; all 65535: 111 / 115 and 85 / 89).
@@ -316,7 +316,7 @@ hipError_t launch_score_d128_g(const int32_t* qs, const int32_t* qm, const float
         return hipGetLastError();
     }
     if (score_takes_mfma(G, qpk, batch * kvh * tokens)) {
-        const int span = score_span(G, qpk, tokens, batch * kvh, !std::is_void_v<QT>, seq.tokens != nullptr);
+        const int span = score_span(G, qpk, tokens, batch * kvh, !std::is_void_v<QT>, seq.tokens != nullptr && batch > 1);
         grid.x = static_cast<unsigned>((tokens + span - 1) / span);
 #define POPKV_SCORE_MFMA(Q)                                                                                             \
     hipLaunchKernelGGL((score_d128_mfma_kernel<G, Q, QT>), grid, dim3(kScoreThreads), 0, stream, qs, qm, ql, qd, q_raw, \
