@@ -461,7 +461,8 @@ __global__ __launch_bounds__(kDenseThreads) void attn_dense_mfma_kernel(
 // Splits of a dense layer: a workgroup per CU in all (a second one per CU
 // only adds its epilogue: 32 query heads over 8 KV heads at 32767 tokens
 // 31.1 us with 256 workgroups, 41.6 with 512; 64 over 8 at 50001 48.1 and
-// 56.7; 32 over 32 at 8191 27.7 and 29.2), of whole tiles and at least one
+// 56.7; 32 over 32 at 8191 27.7 and 29.2; fp32, 64 over 8 at 65536 108.7 and
+// 115.0, 8 over 4 at 16384 19.9 and 20.6), of whole tiles and at least one
 // per wave.
 constexpr int kDenseBlocks = 256;
 constexpr int kDenseLeast = kDenseWaves * kDenseTile;
